@@ -211,11 +211,11 @@ __global__ __launch_bounds__(256) void stage_kernel(StageParams P) {
       const int l = gi & 63;
       const int cks = gi >> 6;  // chunk * NDB + ks
       const int c = cks / SS::NDB, ks = cks - c * SS::NDB;
-      // D > 128: the keys of each 32-key span in attn_wide_kernel's order
+      // D > 256: the keys of each 32-key span in attn_wide_kernel's order
       // (8 (r / 4) + r % 4, then 8 (r / 4) + 4 + r % 4), so that each of its
       // K operands is one whole 16-key chunk
       const int q = 16 * c + (l & 15);
-      const int kq = D > 128 ? 32 * (q >> 5) + 8 * ((q & 15) >> 2) + 4 * ((q >> 4) & 1) + (q & 3) : q;
+      const int kq = D > 256 ? 32 * (q >> 5) + 8 * ((q & 15) >> 2) + 4 * ((q >> 4) & 1) + (q & 3) : q;
       const int j = src_row(j0 + kq);
       x[u] = j >= 0 ? load16(src + int64_t(j) * P.k_ss + 32 * ks + 8 * (l >> 4)) : zero_u32x4();
     }
@@ -420,6 +420,44 @@ struct TileSeq {
   __device__ bool masked(int q) const { return q >= mpos; }
 };
 
+// The tiles of an item of a stream_llm / block_sparse / dense / full head
+// whose rows are the absolute positions a0 .. a1 (list_row: its row of the
+// block lists).  Tiles that need no mask come first, boundary tiles last.
+__device__ inline void item_tiles(const AttnParams& P, int kind, int64_t list_row, int a0, int a1,
+                                  int n_init, int n_local, TileSeq& seq) {
+  const int last_tile = min(a1 >> 6, P.n_kb - 1);
+  // tile t needs no mask for the causal / S_k bounds iff t < Fe
+  const int Fe = min(min((a0 + 1) >> 6, P.s_k >> 6), last_tile + 1);
+  seq.n_kb = P.n_kb;
+  seq.list = nullptr;
+  seq.any = reinterpret_cast<const int32_t*>(P.q);
+  if (kind == KIND_BLOCK) {
+    // canonical list: ascending causal ids, so the boundary ids come last
+    const int cnt = max(0, min(load_uniform(P.cnt + list_row), P.topk_max));
+    const int32_t* list = P.idx + list_row * P.topk_max;
+    int nf = cnt;
+    while (nf > 0 && load_uniform(list + nf - 1) >= Fe) --nf;
+    seq.list = list;
+    seq.set({0, nf, 0, 0, 0}, {nf, cnt, 0, 0, 0}, 1);
+  } else if (kind == KIND_STREAM) {
+    const int lo = min(max(a0 - n_local + 1, 0) >> 6, last_tile + 1);
+    const int nsink = min((min(max(n_init, 0), P.s_k) + 63) >> 6, lo);
+    const int sf = max(0, min(nsink, min(n_init >> 6, Fe)));  // sink tiles below n_init
+    int bf0 = a1 - n_local + 1;                                 // band tiles in every row's band
+    bf0 = bf0 <= 0 ? 0 : (bf0 + 63) >> 6;
+    bf0 = min(max(bf0, lo), last_tile + 1);
+    const int fb_hi = max(bf0, Fe);
+    // full sink, full band | partial sink, band tiles cut by the window
+    // start, diagonal / S_k boundary
+    seq.set({0, bf0, sf, lo, fb_hi}, {sf, fb_hi, nsink, bf0, last_tile + 1}, 2);
+  } else if (kind == KIND_FULL) {
+    const int ff = P.s_k >> 6;  // tiles whose keys are all below S_k
+    seq.set({0, ff, 0, 0, 0}, {ff, P.n_kb, 0, 0, 0}, 1);
+  } else {
+    seq.set({0, Fe, 0, 0, 0}, {Fe, last_tile + 1, 0, 0, 0}, 1);
+  }
+}
+
 template <typename TO>
 __device__ inline void store_out4(TO* dst, float a, float b, float c, float d);
 
@@ -518,49 +556,21 @@ void attn_kernel(AttnParams P) {
     const int off = P.s_k - P.s_q;
     a0 = q0 + off;
     const int a1 = q0 + nrows - 1 + off;
-    const int last_tile = min(a1 >> 6, P.n_kb - 1);
     n_init = P.hd[h].p1;
     n_local = P.hd[h].p2;
-    // tile t needs no mask for the causal / S_k bounds iff t < F
-    const int Fe = min(min((a0 + 1) >> 6, P.s_k >> 6), last_tile + 1);
-
-    seq.n_kb = P.n_kb;
-    seq.list = nullptr;
-    seq.any = reinterpret_cast<const int32_t*>(P.q);
     if constexpr (VS) {
       // this wave's list: unmasked entries, then masked key tiles and
       // gathered vertical tiles (ids n_kb + g), each with its chunk's key bits
       const int64_t lrow = ((int64_t(b) * P.vs_slots + hd_slot) * P.n_qb + bq) * 4 + w;
       const int nf = load_uniform(P.vs_cnt + 2 * lrow);
       const int nt = load_uniform(P.vs_cnt + 2 * lrow + 1);
+      seq.any = reinterpret_cast<const int32_t*>(P.q);
       seq.list = reinterpret_cast<const int32_t*>(P.vs_lists + lrow * P.vs_cap);
       seq.n_kb = P.n_kb + P.nv_pad / kBlock;
       seq.set({0, nf, 0, 0, 0}, {nf, nt, 0, 0, 0}, 1);
-    } else if (kind == KIND_BLOCK) {
-      // canonical list: ascending causal ids, so the boundary ids come last
-      const int64_t base = (int64_t(b) * P.idx_slots + hd_slot) * P.n_qb + bq;
-      const int cnt = max(0, min(load_uniform(P.cnt + base), P.topk_max));
-      const int32_t* list = P.idx + base * P.topk_max;
-      int nf = cnt;
-      while (nf > 0 && load_uniform(list + nf - 1) >= Fe) --nf;
-      seq.list = list;
-      seq.set({0, nf, 0, 0, 0}, {nf, cnt, 0, 0, 0}, 1);
-    } else if (kind == KIND_STREAM) {
-      const int lo = min(max(a0 - n_local + 1, 0) >> 6, last_tile + 1);
-      const int nsink = min((min(max(n_init, 0), P.s_k) + 63) >> 6, lo);
-      const int sf = max(0, min(nsink, min(n_init >> 6, Fe)));  // sink tiles below n_init
-      int bf0 = a1 - n_local + 1;                                 // band tiles in every row's band
-      bf0 = bf0 <= 0 ? 0 : (bf0 + 63) >> 6;
-      bf0 = min(max(bf0, lo), last_tile + 1);
-      const int fb_hi = max(bf0, Fe);
-      // full sink, full band | partial sink, band tiles cut by the window
-      // start, diagonal / S_k boundary
-      seq.set({0, bf0, sf, lo, fb_hi}, {sf, fb_hi, nsink, bf0, last_tile + 1}, 2);
-    } else if (kind == KIND_FULL) {
-      const int ff = P.s_k >> 6;  // tiles whose keys are all below S_k
-      seq.set({0, ff, 0, 0, 0}, {ff, P.n_kb, 0, 0, 0}, 1);
     } else {
-      seq.set({0, Fe, 0, 0, 0}, {Fe, last_tile + 1, 0, 0, 0}, 1);
+      item_tiles(P, kind, (int64_t(b) * P.idx_slots + hd_slot) * P.n_qb + bq, a0, a1, n_init,
+                 n_local, seq);
     }
     total = seq.total;
     mpos = min(seq.mpos, total);
@@ -1045,11 +1055,398 @@ void attn_kernel(AttnParams P) {
 }
 
 // ---------------------------------------------------------------------------
-// Head dims 256 and 512 (the ops zero-pad head dims 129..511 to them).  The
-// same work items and tile walk as attn_kernel; the O of 64 rows x D does
-// not fit one wave, so wave w owns the 16 query rows 16w .. 16w+15 and walks
-// every key of the item's tiles itself (no merge).  Each 32-key span of a
-// tile gives two 16x16x32 QK accumulators whose rows are the keys
+// Head dims 128 and 256, every kind but vertical_and_slash.  At these widths
+// attn_kernel's wave (the O of 64 rows x D) takes more than 256 registers, so
+// one wave runs per SIMD and every item's start and merge are exposed.  Here
+// the four waves of an item share the O instead: wave w scores the 16-key
+// chunk 16w .. 16w+15 of the tile as in attn_kernel, but it accumulates only
+// the output dims 32 NW w .. +32 NW - 1 (NW = D / 128), over all 64 keys.
+// The P of the four chunks pass through LDS in the PV operand's order (8 KB
+// per tile, 16 bytes per lane and access, double-buffered), one barrier per
+// tile; K and V operands still go from L2 straight to registers, each read
+// by one wave.  The running max of a row is common to the four waves, so the
+// output needs no merge: only the row sums meet at the end.
+// Speculative softmax as in attn_kernel; a wave that sees a P sum above
+// 2^15 leaves the tile's stamp in LDS, and after the tile's barrier every
+// wave takes the rare path together (row maxima exchanged through LDS, O and
+// sums rescaled, P written again).
+// Registers: 243 at D = 128 (two waves per SIMD), 426 at D = 256 (one).
+// Whole calls against attn_kernel (D = 128) and a kernel with 16 rows per wave
+// and each tile copied to LDS (D = 256), K in place: dense fp16, 16 heads x
+// 8000 x 128, 358 -> 332 us; fixed block ids, top 16, 8 heads x 32768 x 128,
+// 442 -> 358 us; stream (128, 4096), 8 heads x 16384 x 256, 722 -> 680 us.
+// ---------------------------------------------------------------------------
+template <int D>
+struct SplitShape {
+  static constexpr int NKS = D / 32;  // QK k-steps of 32 dims
+  static constexpr int NDB = D / 32;  // staged V blocks of 32 dims per chunk
+  static constexpr int NW = D / 128;  // output blocks of 32 dims per wave
+};
+
+// Workgroup barrier that orders LDS accesses only: __syncthreads would also
+// wait for the operand loads in flight.
+__device__ inline void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+template <typename T, bool OUT_F32, int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2)))
+void attn_split_kernel(AttnParams P) {
+  using S = SplitShape<D>;
+  constexpr int NKS = S::NKS, NDB = S::NDB, NW = S::NW;
+  static_assert(NW * 128 == D, "whole output blocks per wave");
+  __shared__ __align__(16) u32x4 pbuf[2][4][2][64];  // [parity][chunk][row half][lane]
+  __shared__ float rowmax[4][64];                     // rare path: per wave, rows 0..63
+  __shared__ float2 rowsum[4][64];                    // per wave and lane: sums of its two rows
+  __shared__ int stamp[2];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int lr = lane >> 4;
+  const int lc = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int xcd = blockIdx.x & 7;
+  int hh, bq;
+  if (P.n_hl) {
+    const int r = int(blockIdx.x) >> 3;
+    if (r >= P.xcd_count[xcd]) return;
+    const int g = P.xcd_start[xcd] + r;
+    const int hl = g / P.n_qb;
+    hh = int(P.head_order[hl]);
+    bq = P.n_qb - 1 - (g - hl * P.n_qb);
+  } else {
+    const int BH = P.batch * P.heads;
+    hh = int(blockIdx.x) % BH;
+    if (P.hd[hh % P.heads].kind == KIND_SKIP) return;
+    bq = P.n_qb - 1 - int(blockIdx.x) / BH;
+  }
+  const int b = hh / P.heads;
+  const int h = hh - b * P.heads;
+  const int kvh = h / P.kv_group;
+  const int kind = P.hd[h].kind;
+  const int q0 = bq * kBlock;
+  const int nrows = min(kBlock, P.s_q - q0);
+  const int a0 = q0 + P.s_k - P.s_q;
+  const int n_init = P.hd[h].p1;
+  const int n_local = P.hd[h].p2;
+  TileSeq seq;
+  item_tiles(P, kind, (int64_t(b) * P.idx_slots + P.hd[h].slot) * P.n_qb + bq, a0, a0 + nrows - 1,
+             n_init, n_local, seq);
+  const int total = seq.total;
+  const int mpos = min(seq.mpos, total);
+  const int64_t bk = int64_t(b) * (P.heads / P.kv_group) + kvh;
+  const float vfac = __builtin_amdgcn_ldexpf(1.0f, load_uniform(P.vexp + bk));
+  const bool k_in_place = P.k_in_place;
+  const __amdgpu_buffer_rsrc_t krs =
+      k_in_place
+          ? __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<uint16_t*>(reinterpret_cast<const uint16_t*>(P.k) + b * P.k_sb +
+                                      int64_t(kvh) * P.k_sh),
+                short(0), int(((P.s_k - 1) * P.k_ss + D) * 2), 0x00020000)
+          : __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(P.kt + bk * P.s_pad * D),
+                                              short(0), P.s_pad * D * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(P.vt + bk * P.s_pad * D), short(0), P.s_pad * D * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t qrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(reinterpret_cast<const uint16_t*>(P.q) + b * P.q_sb +
+                            int64_t(h) * P.q_sh + int64_t(q0) * P.q_ss),
+      short(0), int(((nrows - 1) * P.q_ss + D) * 2), 0x00020000);
+  const float c_log2 = P.hd[h].scale_log2;
+  const int arow0 = a0 + lc;
+  const bool is_full = kind == KIND_FULL, is_stream = kind == KIND_STREAM;
+  const int sink_hi = is_stream ? n_init : 0;
+  const int skm1 = P.s_k - 1;
+
+  // operands: K chunk w of a tile (in place or staged, see attn_kernel), V of
+  // all four chunks at this wave's dims
+  const uint32_t lane_off = 16u * lane;
+  const uint32_t k_row_bytes = uint32_t(P.k_ss) * 2u;
+  const uint32_t k_lane = k_in_place ? uint32_t(lc) * k_row_bytes + 16u * lr : lane_off;
+  const uint32_t k_cv = k_in_place ? 16u * k_row_bytes : 0u;
+  const int k_cs = k_in_place ? 0 : NKS * 1024;
+  const int k_kss = k_in_place ? 64 : 1024;
+  auto load_k = [&](int t, u32x4 (&kr)[NKS], bool drop) INLINE {
+    const int c = 4 * t + w;
+    const uint32_t vo = (k_lane + uint32_t(c) * k_cv) | (drop ? 0x80000000u : 0u);
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks)
+      kr[ks] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(krs, vo, c * k_cs + k_kss * ks, 0));
+  };
+  auto load_v = [&](int t, u32x4 (&vr)[NW][4], bool drop) INLINE {
+    const uint32_t vo = lane_off | (drop ? 0x80000000u : 0u);
+#pragma unroll
+    for (int nw = 0; nw < NW; ++nw)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        vr[nw][c] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                       vrs, vo, ((4 * t + c) * NDB + w * NW + nw) * 1024, 0));
+  };
+
+  u32x4 qb[4][NKS];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const uint32_t roff = uint32_t((16 * g + lc) * P.q_ss * 2 + 16 * lr);
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks)
+      qb[g][ks] =
+          __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(qrs, roff, 64 * ks, 0));
+  }
+  if constexpr (D > 128) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) asm volatile("" : "+a"(qb[g][ks]));
+  }
+  f32x16 o[NW][2];
+#pragma unroll
+  for (int nw = 0; nw < NW; ++nw)
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[nw][hf][i] = 0.0f;
+  float m_g[4], l_g[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    m_g[g] = -1e30f;
+    l_g[g] = 0.0f;
+  }
+  if (tid < 2) stamp[tid] = -1;
+
+  // k-steps [ks0, ks1) of a chunk's scores
+  auto qk = [&](const u32x4 (&kr)[NKS], f32x4 (&s)[4], int ks0, int ks1) INLINE {
+    if (ks0 == 0)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) s[g] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int ks = ks0; ks < ks1; ++ks)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) s[g] = mfma_qk<T>(kr[ks], qb[g][ks], s[g]);
+  };
+  // visible iff j <= key_hi and (j >= band_lo or j < sink_hi)
+  auto mask = [&](f32x4 (&s)[4], int t) INLINE {
+    const int jb = t * kBlock + 16 * w + 4 * lr;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int ar = arow0 + 16 * g;
+      const int key_hi = is_full ? skm1 : min(ar, skm1);
+      const int band_lo = is_stream ? ar - n_local + 1 : 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = jb + i;
+        const bool vis = (j <= key_hi) & ((j >= band_lo) | (j < sink_hi));
+        s[g][i] = vis ? s[g][i] : -__builtin_inff();
+      }
+    }
+  };
+  // P of a tile's chunk from its scores, into LDS; ps = the lane's sums.
+  // Returns true when some sum exceeds 2^15.
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  auto softmax = [&](const f32x4 (&s)[4], float (&ps)[4], int par) INLINE -> bool {
+    uint32_t pk[4][2];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4 e;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        e[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[g][i], c_log2, -m_g[g]));
+      ps[g] = (e[0] + e[1]) + (e[2] + e[3]);
+      pk[g][0] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{e[0], e[1]}, h2));
+      pk[g][1] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{e[2], e[3]}, h2));
+    }
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      uint32_t x0 = pk[2 * hf][0], y0 = pk[2 * hf + 1][0];
+      uint32_t x1 = pk[2 * hf][1], y1 = pk[2 * hf + 1][1];
+      swap16(x0, y0);
+      swap16(x1, y1);
+      pbuf[par][w][hf][lane] = u32x4{x0, x1, y0, y1};
+    }
+    return __ballot(fmaxf(fmaxf(ps[0], ps[1]), fmaxf(ps[2], ps[3])) > kPCheck) != 0;
+  };
+  auto read_p = [&](u32x4 (&pb)[2][4], int par) INLINE {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) pb[hf][c] = pbuf[par][c][hf][lane];
+  };
+  auto pv = [&](const u32x4 (&pb)[2][4], const u32x4 (&vr)[NW][4]) INLINE {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int nw = 0; nw < NW; ++nw)
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) o[nw][hf] = mfma_pv(vr[nw][c], pb[hf][c], o[nw][hf]);
+  };
+  // Rare path, every wave together: raise the running maxima to the tile's
+  // row maxima, rescale O and the row sums, write the tile's P again.
+  auto rescale = [&](const f32x4 (&s)[4], float (&ps)[4], u32x4 (&pb)[2][4], int par) INLINE {
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      const f32x4 a = s[2 * hf], c = s[2 * hf + 1];
+      float m0 = fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3]));
+      float m1 = fmaxf(fmaxf(c[0], c[1]), fmaxf(c[2], c[3]));
+      swap32(m0, m1);
+      float x = fmaxf(m0, m1), y = x;
+      swap16(x, y);
+      float g0 = fmaxf(x, y), g1 = g0;
+      swap32(g0, g1);  // g0: group 2 hf in every lane row, g1: group 2 hf + 1
+      rowmax[w][32 * hf + lc] = g0;
+      rowmax[w][32 * hf + 16 + lc] = g1;
+    }
+    lds_barrier();  // and every wave has read the tile's old P
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      auto raise = [&](int g) INLINE -> float {
+        const int r = 16 * g + lc;
+        const float top =
+            fmaxf(fmaxf(rowmax[0][r], rowmax[1][r]), fmaxf(rowmax[2][r], rowmax[3][r]));
+        const float n = fmaxf(m_g[g], top * c_log2 - kPBias);
+        const float al = __builtin_amdgcn_exp2f(m_g[g] - n);
+        m_g[g] = n;
+        l_g[g] *= al;
+        return al;
+      };
+      const float al0 = raise(2 * hf), al1 = raise(2 * hf + 1);
+      const float ab = (lr & 1) ? al1 : al0;
+#pragma unroll
+      for (int nw = 0; nw < NW; ++nw) {
+        // D > 128: O lives in accumulation registers; taken out and put back
+        // here, or the copies land in front of the branch, on every tile
+        if constexpr (D > 128) asm volatile("" : "+a"(o[nw][hf]));
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[nw][hf][i] *= ab;
+        if constexpr (D > 128) asm volatile("" : "+a"(o[nw][hf]));
+      }
+    }
+    softmax(s, ps, par);
+    lds_barrier();
+    read_p(pb, par);
+  };
+
+  // Iteration p: the tile's P become visible (barrier), QK of p + 1, PV of p,
+  // softmax of p + 1 under it.  K of p + 2 is requested once QK of p + 1 is
+  // issued, V of p + 1 once PV of p is.  One wave per SIMD (D = 256): the
+  // barrier and the LDS reads are pinned between two halves of QK, the first
+  // covering the waves' skew, the second the reads' latency (585 against
+  // 627 us on the launch below; no difference at D = 128, where the second
+  // workgroup on the CU covers them).
+  constexpr bool PIN = D > 128;
+  constexpr int KH = PIN ? NKS / 2 : 0;
+  u32x4 kr[NKS], vr[NW][4];
+  f32x4 sA[4], sB[4];
+  float pA[4], pB[4];
+  int t1 = 0, t2 = 0;
+  TileSeq::Pending pn{0, 0};
+  auto step = [&](auto masked, auto last, f32x4 (&s)[4], float (&ps)[4], f32x4 (&sn)[4],
+                  float (&pns)[4], int par, int p) INLINE {
+    constexpr bool MT = decltype(masked)::value, LAST = decltype(last)::value;
+    if constexpr (!LAST) qk(kr, sn, 0, KH);
+    if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
+    lds_barrier();
+    const int flag = stamp[par];
+    u32x4 pb[2][4];
+    read_p(pb, par);
+    if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
+    int t3 = 0;
+    if constexpr (!LAST) {
+      t3 = seq.template finish<false>(pn);
+      pn = seq.fetch(p + 4);
+      qk(kr, sn, KH, NKS);
+      load_k(t2, kr, p + 2 >= total);
+    }
+    if constexpr (PIN) {  // keep the reads here: they would sink past the branch
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(pb[hf][c]));
+    }
+    if (__builtin_amdgcn_readfirstlane(flag) == p) rescale(s, ps, pb, par);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) l_g[g] += ps[g];
+    pv(pb, vr);
+    if constexpr (!LAST) {
+      load_v(t1, vr, false);
+      if constexpr (MT) mask(sn, t1);
+      if (softmax(sn, pns, par ^ 1) && lane == 0) stamp[par ^ 1] = p + 1;
+      t1 = t2;
+      t2 = t3;
+    }
+  };
+  const std::integral_constant<bool, false> no{};
+  const std::integral_constant<bool, true> yes{};
+  auto run = [&](auto masked, int p0, int p1) INLINE {
+    int p = p0;
+    if ((p & 1) && p < p1) {
+      step(masked, no, sB, pB, sA, pA, 1, p);
+      ++p;
+    }
+    for (; p + 1 < p1; p += 2) {
+      step(masked, no, sA, pA, sB, pB, 0, p);
+      step(masked, no, sB, pB, sA, pA, 1, p + 1);
+    }
+    if (p < p1) step(masked, no, sA, pA, sB, pB, 0, p);
+  };
+  if (total > 0) {
+    const TileSeq::Pending p0 = seq.fetch(0), p1 = seq.fetch(1), p2 = seq.fetch(2);
+    const int t0 = seq.template finish<false>(p0);
+    t1 = seq.template finish<false>(p1);
+    t2 = seq.template finish<false>(p2);
+    load_k(t0, kr, false);
+    load_v(t0, vr, false);
+    pn = seq.fetch(3);
+    qk(kr, sA, 0, NKS);
+    load_k(t1, kr, total < 2);
+    mask(sA, t0);
+    __syncthreads();  // stamps initialised
+    if (softmax(sA, pA, 0) && lane == 0) stamp[0] = 0;
+    // iteration p computes the scores of p + 1
+    run(no, 0, max(mpos - 1, 0));
+    run(yes, max(mpos - 1, 0), total - 1);
+    if ((total - 1) & 1) step(no, yes, sB, pB, sA, pA, 1, total - 1);
+    else step(no, yes, sA, pA, sB, pB, 0, total - 1);
+  }
+
+  // row sums of the four chunks; O^T block: lane l holds floats 4 v .. 4 v + 3
+  // = dims 8 v + 4 (l / 32) .. +3 of row 32 hf + l % 32
+  float l_b[2];
+  lanes_to_blocks(reduce_rows(l_g[0], l_g[1], l_g[2], l_g[3], RowSum()), l_b);
+  rowsum[w][lane] = float2{l_b[0], l_b[1]};
+  __syncthreads();
+  const float2 r0 = rowsum[0][lane], r1 = rowsum[1][lane], r2 = rowsum[2][lane],
+               r3 = rowsum[3][lane];
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    const float lt = hf ? (r0.y + r1.y) + (r2.y + r3.y) : (r0.x + r1.x) + (r2.x + r3.x);
+    const float inv = lt > 0.0f ? vfac / lt : 0.0f;
+    const int row = q0 + 32 * hf + (lane & 31);
+    if (row >= P.s_q) continue;
+    const int64_t obase = b * P.o_sb + int64_t(h) * P.o_sh + int64_t(row) * P.o_ss;
+#pragma unroll
+    for (int nw = 0; nw < NW; ++nw)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int d = 32 * (w * NW + nw) + 8 * v + 4 * (lane >> 5);
+        const f32x16& x = o[nw][hf];
+        if constexpr (OUT_F32) {
+          store_out4<float>(reinterpret_cast<float*>(P.o) + obase + d, x[4 * v] * inv,
+                            x[4 * v + 1] * inv, x[4 * v + 2] * inv, x[4 * v + 3] * inv);
+        } else {
+          store_out4_16<T>(reinterpret_cast<uint16_t*>(P.o) + obase + d, x[4 * v] * inv,
+                           x[4 * v + 1] * inv, x[4 * v + 2] * inv, x[4 * v + 3] * inv);
+        }
+      }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Head dim 512 (the ops zero-pad head dims 257..511 to it).  The same work
+// items and tile walk; neither the Q of 64 rows nor the O of attn_split_kernel
+// fits one wave's registers at this width, so wave w owns the 16 query rows
+// 16w .. 16w+15 and walks every key of the item's tiles itself (no merge).
+// Each 32-key span of a tile gives two 16x16x32 QK accumulators whose rows are the keys
 //   A: 8 (r / 4) + (r % 4),   B: 8 (r / 4) + 4 + (r % 4)   (r = accumulator row)
 // (the staging writes K of this head dim in that key order, so each QK
 // operand is one contiguous staged 16-key chunk), so lane l holds keys
@@ -1057,12 +1454,14 @@ void attn_kernel(AttnParams P) {
 // operand of the 16x16x32 PV product as they stand.  V comes from the staged
 // 32x32x16 operand layout, one 16-byte granule per lane.  The row max is
 // exact per tile (O rescaled when it grows), P biased to 2^kPBias like
-// attn_kernel; fully masked rows give 0.  At D = 512 one wave per SIMD (the
-// O accumulators, a K chunk and a V span take about 500 registers).
+// attn_kernel; fully masked rows give 0.  One wave per SIMD (the O
+// accumulators, a K chunk and a V span take about 500 registers); every wave
+// reads the operands from L2 itself (a 128 KB LDS tile would leave one
+// workgroup per CU, measured slower).
 template <typename T, bool OUT_F32, int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D > 256 ? 1 : 2)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1)))
 void attn_wide_kernel(AttnParams P) {
-  static_assert(D == 256 || D == 512, "wide head dims");
+  static_assert(D == 512, "wide head dim");
   constexpr int NKS = D / 32;  // QK k-steps
   constexpr int NDO = D / 16;  // PV output blocks of 16 dims
   constexpr int NDB = D / 32;  // staged V blocks of 32 dims per 16-key chunk
@@ -1152,18 +1551,7 @@ void attn_wide_kernel(AttnParams P) {
   float m = -1e30f;  // running (biased) max of the row in scaled log2 units
   float l = 0.0f;    // this lane's share of the row sum
 
-  // At D = 256 the workgroup copies each tile's staged K and V into LDS (the
-  // four waves read the same operands: each line then leaves L2 once per
-  // workgroup instead of once per wave; 64 KB, two workgroups per CU); at
-  // D = 512 every wave reads them from L2 itself (a 128 KB tile would leave
-  // one workgroup per CU, measured slower).
-  constexpr bool SHARED = D == 256;
-  constexpr int TILE_BYTES = 64 * D * 2;    // one tile of staged K (or V)
-  constexpr int G = TILE_BYTES / 16 / 256;  // 16-byte granules per thread and plane
-  __shared__ __align__(16) unsigned char sm[SHARED ? 2 * TILE_BYTES : 16];
-  auto lds16 = [&](int off) INLINE -> u32x4 {
-    return *reinterpret_cast<const u32x4*>(sm + off);
-  };
+  constexpr int TILE_BYTES = 64 * D * 2;  // one tile of staged K (or V)
   // K operand of virtual chunk vc (span vc / 2, half vc % 2) of tile t: the
   // staged chunk 4t + vc, whose row r is key 32 (vc / 2) + 8 (r / 4) +
   // 4 (vc % 2) + r % 4 of the tile; lane (lc, lr) of k-step ks holds
@@ -1171,12 +1559,8 @@ void attn_wide_kernel(AttnParams P) {
   auto load_k = [&](int t, int vc, u32x4 (&kr)[NKS]) INLINE {
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
-      if constexpr (SHARED) {
-        kr[ks] = lds16((vc * NKS + ks) * 1024 + lane * 16);
-      } else {
-        const uint32_t vo = uint32_t((4 * t + vc) * NKS * 1024 + lane * 16);
-        kr[ks] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(krs, vo, 1024 * ks, 0));
-      }
+      const uint32_t vo = uint32_t((4 * t + vc) * NKS * 1024 + lane * 16);
+      kr[ks] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(krs, vo, 1024 * ks, 0));
     }
   };
   auto qk = [&](const u32x4 (&kr)[NKS]) INLINE -> f32x4 {
@@ -1193,34 +1577,14 @@ void attn_wide_kernel(AttnParams P) {
 #pragma unroll
     for (int db = 0; db < NDO; ++db) {
       const int go = ((c * NDB + (db >> 1)) * 64 + 32 * (lr & 1) + 16 * (db & 1) + lc) * 16;
-      if constexpr (SHARED) {
-        vr[db] = lds16(TILE_BYTES + go);
-      } else {
-        vr[db] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(vrs, uint32_t(t * TILE_BYTES + go), 0, 0));
-      }
+      vr[db] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(vrs, uint32_t(t * TILE_BYTES + go), 0, 0));
     }
   };
 
   u32x4 k0[NKS];
   for (int p = 0; p < total; ++p) {
     const int t = seq.template finish<false>(seq.fetch(p));
-    if constexpr (SHARED) {
-      __syncthreads();  // every wave has read the previous tile
-      u32x4 gk[G], gv[G];
-#pragma unroll
-      for (int u = 0; u < G; ++u) {
-        const uint32_t go = uint32_t((tid + 256 * u) * 16);
-        gk[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(krs, go, t * TILE_BYTES, 0));
-        gv[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(vrs, go, t * TILE_BYTES, 0));
-      }
-#pragma unroll
-      for (int u = 0; u < G; ++u) {
-        *reinterpret_cast<u32x4*>(sm + (tid + 256 * u) * 16) = gk[u];
-        *reinterpret_cast<u32x4*>(sm + TILE_BYTES + (tid + 256 * u) * 16) = gv[u];
-      }
-      __syncthreads();
-    }
     // scores of the tile: s[kh][ab] (lane: keys 8 lr + 4 ab + i of span kh)
     f32x4 s[2][2];
     u32x4 vr[NDO];  // V of span 0, requested under the last QK
@@ -1304,14 +1668,25 @@ void attn_wide_kernel(AttnParams P) {
   }
 }
 
+// Workgroups of a launch of one item each: the longest XCD range on every XCD.
+static int64_t item_grid(const AttnParams& p) {
+  if (!p.n_hl) return int64_t(p.n_qb) * p.batch * p.heads;
+  int longest = 0;
+  for (int x = 0; x < 8; ++x) longest = p.xcd_count[x] > longest ? p.xcd_count[x] : longest;
+  return 8 * int64_t(longest);
+}
+
+template <typename T, bool OUT_F32, int D>
+static hipError_t launch_split_t(const AttnParams& p, hipStream_t st) {
+  const int64_t items = item_grid(p);
+  if (items == 0) return hipSuccess;
+  hipLaunchKernelGGL((attn_split_kernel<T, OUT_F32, D>), dim3(uint32_t(items)), dim3(256), 0, st, p);
+  return hipGetLastError();
+}
+
 template <typename T, bool OUT_F32, int D>
 static hipError_t launch_wide_t(const AttnParams& p, hipStream_t st) {
-  int64_t items = int64_t(p.n_qb) * p.batch * p.heads;
-  if (p.n_hl) {
-    int longest = 0;
-    for (int x = 0; x < 8; ++x) longest = p.xcd_count[x] > longest ? p.xcd_count[x] : longest;
-    items = 8 * int64_t(longest);
-  }
+  const int64_t items = item_grid(p);
   if (items == 0) return hipSuccess;
   hipLaunchKernelGGL((attn_wide_kernel<T, OUT_F32, D>), dim3(uint32_t(items)), dim3(256), 0, st, p);
   return hipGetLastError();
@@ -1319,12 +1694,7 @@ static hipError_t launch_wide_t(const AttnParams& p, hipStream_t st) {
 
 template <typename T, bool OUT_F32, int D, bool VS>
 static hipError_t launch_attn_t(const AttnParams& p, hipStream_t st) {
-  int64_t items = int64_t(p.n_qb) * p.batch * p.heads;
-  if (p.n_hl) {
-    int longest = 0;
-    for (int x = 0; x < 8; ++x) longest = p.xcd_count[x] > longest ? p.xcd_count[x] : longest;
-    items = 8 * int64_t(longest);
-  }
+  int64_t items = item_grid(p);
   if (VS) {
     // persistent grid: the resident workgroups of every XCD (2 per CU at
     // two waves per SIMD, 1 for D = 128), capped by the work
@@ -1342,11 +1712,17 @@ static hipError_t launch_attn_t(const AttnParams& p, hipStream_t st) {
 
 template <typename T, bool OUT_F32, bool VS>
 static hipError_t launch_attn_d(const AttnParams& p, int D, hipStream_t st) {
-  if (D == 256) return VS ? hipErrorInvalidValue : launch_wide_t<T, OUT_F32, 256>(p, st);
+  if constexpr (!VS) {
+    if (D == 128) return launch_split_t<T, OUT_F32, 128>(p, st);
+    if (D == 256) return launch_split_t<T, OUT_F32, 256>(p, st);
+  }
   if (D == 512) return VS ? hipErrorInvalidValue : launch_wide_t<T, OUT_F32, 512>(p, st);
   if (D == 64) return launch_attn_t<T, OUT_F32, 64, VS>(p, st);
   if (D == 96) return launch_attn_t<T, OUT_F32, 96, VS>(p, st);
-  return launch_attn_t<T, OUT_F32, 128, VS>(p, st);
+  if constexpr (VS) {
+    if (D == 128) return launch_attn_t<T, OUT_F32, 128, VS>(p, st);
+  }
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_attention(const AttnParams& p, int dtype, int out_dtype, int D,
