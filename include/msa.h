@@ -194,8 +194,9 @@ int msa_layer_attention(const msa_tensor4* q, const msa_tensor4* k,
  * caller can time the attention kernel alone, or reuse one staging):
  *   msa_stage_kv: V [B][H_kv][S_k][D] -> MFMA operand order in the
  *                workspace (msa_attention_workspace_bytes bytes), and K too
- *                when the attention kernel cannot read it in place (rows
- *                that overlap, row stride < D, or one kv head's padded rows
+ *                when the attention kernel does not read it in place (a row
+ *                stride that is not an odd multiple of 64 bytes, rows that
+ *                overlap, row stride < D, or one kv head's padded rows
  *                spanning more than 2^31 bytes); k and v have the same shape
  *                and dtype;
  *   msa_layer_attention_staged: same arguments and checks as

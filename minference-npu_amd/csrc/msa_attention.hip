@@ -1071,10 +1071,12 @@ void attn_kernel(AttnParams P) {
 // wave takes the rare path together (row maxima exchanged through LDS, O and
 // sums rescaled, P written again).
 // Registers: 243 at D = 128 (two waves per SIMD), 426 at D = 256 (one).
-// Whole calls against attn_kernel (D = 128) and a kernel with 16 rows per wave
-// and each tile copied to LDS (D = 256), K in place: dense fp16, 16 heads x
-// 8000 x 128, 358 -> 332 us; fixed block ids, top 16, 8 heads x 32768 x 128,
-// 442 -> 358 us; stream (128, 4096), 8 heads x 16384 x 256, 722 -> 680 us.
+// Bound by the waits between the phases of a tile (MFMA busy 46 % of the
+// cycles at D = 128, 1.87 GHz).  With the staged K (k_in_place in msa_abi.hip),
+// whole calls against attn_kernel (D = 128) and a kernel with 16 rows per wave
+// and each tile copied to LDS (D = 256): dense fp16, 16 heads x 8000 x 128,
+// 362 -> 310 us; one 16K layer of 32 heads on 8 kv heads x 128, 1543 ->
+// 1254 us; stream (128, 4096), 8 heads x 16384 x 256, 728 -> 597 us.
 // ---------------------------------------------------------------------------
 template <int D>
 struct SplitShape {
