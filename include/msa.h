@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MSA_ABI_VERSION 12
+#define MSA_ABI_VERSION 13
 
 /* status codes (negative: validation, nothing launched) */
 #define MSA_OK 0
@@ -353,6 +353,18 @@ int msa_decode_attention_noalloc(const msa_tensor4* q, const msa_tensor4* k,
 int msa_rope_qk(const msa_tensor4* q, const msa_tensor4* k, const msa_tensor4* cos,
                 const msa_tensor4* sin, const msa_tensor4* q_out, const msa_tensor4* k_out,
                 msa_stream_t stream);
+
+/* Rounding of n (1..4) float32 tensors to fp16 (nearest even), one launch:
+ * the inputs of ops called with float32 tensors (the reference's CPU paths
+ * take them, minference/ops/streaming_kernel_npu.py:138-144).  *flag (device
+ * memory, or host memory the device can write; zeroed by the caller) becomes
+ * 1 when a finite value lies beyond fp16's range, and is not written
+ * otherwise.
+ *   src[i] float32 [B][H][S][D]: D % 8 == 0 and contiguous, rows 16-byte aligned
+ *   dst[i] fp16, the same sizes, contiguous
+ * (arrays of n descriptors on the host; at most 2^34 elements each) */
+int msa_round_f32(const msa_tensor4* src, const msa_tensor4* dst, int32_t n, int32_t* flag,
+                  msa_stream_t stream);
 
 #ifdef __cplusplus
 }

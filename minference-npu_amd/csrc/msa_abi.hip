@@ -1004,4 +1004,41 @@ int msa_rope_qk(const msa_tensor4* q, const msa_tensor4* k, const msa_tensor4* c
   return e == hipSuccess ? MSA_OK : int(e);
 }
 
+int msa_round_f32(const msa_tensor4* src, const msa_tensor4* dst, int32_t n, int32_t* flag,
+                  msa_stream_t stream) {
+  if (!src || !dst || !flag) return MSA_E_NULL;
+  if (n < 1 || n > kRoundMax) return MSA_E_RANK;
+  RoundParams rp;
+  memset(&rp, 0, sizeof(rp));
+  rp.flag = flag;
+  for (int i = 0; i < n; ++i) {
+    const msa_tensor4 &a = src[i], &b = dst[i];
+    if (!a.data || !b.data) return MSA_E_NULL;
+    int64_t total = 1;
+    for (int k = 3; k >= 0; --k) {
+      if (a.size[k] <= 0 || a.size[k] != b.size[k]) return MSA_E_RANK;
+      if (a.size[k] > 1 && b.stride[k] != total) return MSA_E_ALIGN;  // dst contiguous
+      if (a.size[k] > (int64_t(1) << 34) / total) return MSA_E_SEQ;
+      total *= a.size[k];
+    }
+    if (a.dtype != MSA_DTYPE_FP32 || b.dtype != MSA_DTYPE_FP16) return MSA_E_DTYPE;
+    if (a.size[3] % 8 != 0) return MSA_E_HEAD_DIM;
+    if (a.stride[3] != 1 || ((reinterpret_cast<uintptr_t>(a.data) |
+                              reinterpret_cast<uintptr_t>(b.data)) & 15u) != 0)
+      return MSA_E_ALIGN;
+    for (int k = 0; k < 3; ++k)
+      if (a.size[k] > 1 && a.stride[k] % 4 != 0) return MSA_E_ALIGN;
+    RoundTensor& t = rp.t[i];
+    t.src = static_cast<const float*>(a.data);
+    t.dst = static_cast<uint16_t*>(b.data);
+    t.sb = a.stride[0]; t.sh = a.stride[1]; t.ss = a.stride[2];
+    t.h = uint32_t(a.size[1]);
+    t.s = uint32_t(a.size[2]);
+    t.upr = uint32_t(a.size[3] / 8);
+    t.units = uint32_t(total / 8);
+  }
+  const hipError_t e = launch_round(rp, n, reinterpret_cast<hipStream_t>(stream));
+  return e == hipSuccess ? MSA_OK : int(e);
+}
+
 }  // extern "C"

@@ -219,6 +219,20 @@ struct RopeParams {
   int batch, heads, kv_heads, s, rot, half, n_pair, n_pass;
 };
 
+// float32 tensors rounded to fp16 in one launch (round_f16_kernel): source
+// strides in elements, contiguous fp16 outputs.
+constexpr int kRoundMax = 4;
+struct RoundTensor {
+  const float* src;
+  uint16_t* dst;
+  int64_t sb, sh, ss;
+  uint32_t h, s, upr, units;  // heads, rows per head, 8-element units per row and in all
+};
+struct RoundParams {
+  RoundTensor t[kRoundMax];
+  int32_t* flag;  // set to 1 when a finite value lies beyond fp16's range
+};
+
 // Widest rotary part msa_rope_qk takes (its cos/sin rows are staged in LDS).
 constexpr int kRopeMaxRot = 256;
 
@@ -238,6 +252,7 @@ hipError_t launch_attention_vs(const AttnParams& p, int dtype, int out_dtype, in
                                hipStream_t st);
 hipError_t launch_vs_build(const VsBuildParams& p, int n_bs, hipStream_t st);
 hipError_t launch_vs_estimate(const VsEstParams& p, int dtype, int D, hipStream_t st);
+hipError_t launch_round(const RoundParams& p, int n, hipStream_t st);
 hipError_t launch_rope(const RopeParams& p, int dtype, hipStream_t st);
 
 }  // namespace msa

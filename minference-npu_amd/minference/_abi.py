@@ -53,7 +53,7 @@ MSA_ESTIMATE_SELECT_ONLY = 8
 
 MSA_MAX_HEADS = 128
 MSA_BLOCK = 64
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 _DTYPE_CODE = {
     torch.bfloat16: MSA_DTYPE_BF16,
@@ -81,6 +81,7 @@ EXPORTED_SYMBOLS = (
     "msa_vs_estimate_workspace_bytes",
     "msa_vs_estimate",
     "msa_rope_qk",
+    "msa_round_f32",
 )
 
 
@@ -242,6 +243,11 @@ def load_library() -> ctypes.CDLL:
         ]
         lib.msa_rope_qk.restype = ctypes.c_int
         lib.msa_rope_qk.argtypes = [ctypes.POINTER(MsaTensor4)] * 6 + [ctypes.c_void_p]
+        lib.msa_round_f32.restype = ctypes.c_int
+        lib.msa_round_f32.argtypes = [
+            ctypes.POINTER(MsaTensor4), ctypes.POINTER(MsaTensor4), ctypes.c_int32,
+            ctypes.c_void_p, ctypes.c_void_p,
+        ]
         ver = lib.msa_abi_version()
         if ver != ABI_VERSION:
             raise ImportError(f"libmsa ABI version {ver} != expected {ABI_VERSION}")
@@ -339,6 +345,30 @@ def rope_qk(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tens
     ds = [tensor4(t) for t in (q, k, cos, sin, q_out, k_out)]
     check(load_library().msa_rope_qk(*[ctypes.byref(d) for d in ds],
                                      current_stream_handle(q.device)))
+
+
+ROUND_MAX = 4  # float32 tensors one msa_round_f32 launch takes
+
+
+def round_f32_supported(ts: Sequence[torch.Tensor]) -> bool:
+    """True when msa_round_f32 takes these float32 tensors: 1 to 4 non-empty
+    4-D GPU tensors with 16-byte aligned rows of a multiple of 8 elements."""
+    return 1 <= len(ts) <= ROUND_MAX and all(
+        t.is_cuda and t.device == ts[0].device and t.dim() == 4 and 0 < t.numel() <= 1 << 34
+        and t.shape[3] % 8 == 0 and t.stride(3) == 1 and t.data_ptr() % 16 == 0
+        and not any(t.stride(i) % 4 for i in range(3) if t.shape[i] > 1) for t in ts)
+
+
+def round_f32(ts: Sequence[torch.Tensor], flag: torch.Tensor) -> list:
+    """Launch msa_round_f32 on the current stream: the fp16 roundings of the
+    float32 tensors ``ts``, contiguous; ``flag`` (one zeroed int32 the device
+    can write) becomes 1 when a finite value lies beyond fp16's range."""
+    outs = [torch.empty(t.shape, dtype=torch.float16, device=t.device) for t in ts]
+    n = len(ts)
+    src, dst = (MsaTensor4 * n)(*map(tensor4, ts)), (MsaTensor4 * n)(*map(tensor4, outs))
+    check(load_library().msa_round_f32(src, dst, n, flag.data_ptr(),
+                                       current_stream_handle(ts[0].device)))
+    return outs
 
 
 def workspace(nbytes: int, device: torch.device) -> torch.Tensor:

@@ -42,7 +42,9 @@ def accepts_float32(names: Sequence[str], has_out: bool = True):
     fp32 (minference/ops/streaming_kernel_npu.py:138-144,
     minference/ops/block_sparse_kernel_npu.py:340-348); here float32 inputs
     get the 16-bit kernels' arithmetic on their roundings.  Inputs of other
-    dtypes go to the op unchanged (bf16 / fp16, or its dtype error)."""
+    dtypes go to the op unchanged (bf16 / fp16, or its dtype error).
+    GPU tensors that msa_round_f32 takes are rounded and range-checked by that
+    one launch, others by torch ops."""
 
     def wrap(fn):
         sig = inspect.signature(fn)
@@ -53,9 +55,6 @@ def accepts_float32(names: Sequence[str], has_out: bool = True):
             ts = [ba.arguments.get(n) for n in names]
             if not all(isinstance(t, torch.Tensor) and t.dtype == torch.float32 for t in ts):
                 return fn(*args, **kwargs)
-            dt = sixteen_bit_dtype(ts)
-            for n, t in zip(names, ts):
-                ba.arguments[n] = t.to(dt)
             if has_out:
                 out = ba.arguments.get("out")
                 if out is None:
@@ -63,7 +62,33 @@ def accepts_float32(names: Sequence[str], has_out: bool = True):
                                                       device=ts[0].device)
                 elif out.dtype != torch.float32:
                     raise ValueError(f"out must be float32 for float32 inputs, got {out.dtype}")
-            return fn(*ba.args, **ba.kwargs)
+            if not _abi.round_f32_supported(ts):
+                dt = sixteen_bit_dtype(ts)
+                ba.arguments.update(zip(names, (t.to(dt) for t in ts)))
+                return fn(*ba.args, **ba.kwargs)
+            # fp16 roundings and the range check in one launch; the op is
+            # queued behind it and runs again on bf16 roundings in the rare
+            # case the check fails (the host waits for the check only, so the
+            # GPU never idles for it)
+            flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+            with torch.cuda.device(ts[0].device):
+                rounded = _abi.round_f32(ts, flag)
+                checked = torch.cuda.Event()
+                checked.record()
+            out = ba.arguments.get("out")
+            aliased = has_out and any(
+                out.untyped_storage().data_ptr() == t.untyped_storage().data_ptr() for t in ts)
+            if aliased:  # the op would write over what a second run reads
+                checked.synchronize()
+                if int(flag[0]):
+                    rounded = [t.to(torch.bfloat16) for t in ts]
+            ba.arguments.update(zip(names, rounded))
+            result = fn(*ba.args, **ba.kwargs)
+            checked.synchronize()
+            if int(flag[0]) and not aliased:
+                ba.arguments.update(zip(names, (t.to(torch.bfloat16) for t in ts)))
+                result = fn(*ba.args, **ba.kwargs)
+            return result
 
         return inner
 
