@@ -842,7 +842,7 @@ int msa_layer_attention_ex(const msa_tensor4* q, const msa_tensor4* k, const msa
 // decode
 // ---------------------------------------------------------------------------
 // Key splits of one decode call: about 2048 workgroups in all, at least 64
-// keys each.
+// keys each (one head per workgroup).
 static void decode_split(int64_t bh, int64_t s_k, int& n_split, int& chunk) {
   int64_t ns = (kDecodeMaxSplit + bh - 1) / bh;
   ns = std::max<int64_t>(1, std::min<int64_t>(ns, cdiv(s_k, 64)));
@@ -850,6 +850,19 @@ static void decode_split(int64_t bh, int64_t s_k, int& n_split, int& chunk) {
   ch = cdiv(ch, 64) * 64;
   n_split = int(cdiv(s_k, ch));
   chunk = int(ch);
+}
+
+// Key splits of a grouped decode (several query heads per workgroup): about
+// 512 workgroups, two per CU (1024 and 2048 measured the same on 8 x 32 heads
+// on 8 x 16384 keys and leave more to merge), whole 128-key rounds of the four
+// waves, and no more splits than the workspace of decode_split holds.
+static void decode_group_split(int64_t bh, int64_t tiles, int64_t s_k, int& n_split, int& chunk) {
+  int ns, ch;
+  decode_split(bh, s_k, ns, ch);
+  const int64_t want = std::max<int64_t>(1, cdiv(512, tiles));
+  const int64_t c = cdiv(std::max<int64_t>(ch, cdiv(s_k, want)), 128) * 128;
+  chunk = int(c);
+  n_split = int(cdiv(s_k, c));
 }
 
 size_t msa_decode_workspace_bytes(int64_t batch, int64_t heads, int64_t s_k, int32_t head_dim) {
@@ -897,7 +910,8 @@ int msa_decode_attention(const msa_tensor4* q, const msa_tensor4* k, const msa_t
   dp.heads = int(H);
   dp.kv_group = int(H / Hkv);
   dp.s_k = int(Sk);
-  decode_split(B * H, Sk, dp.n_split, dp.chunk);
+  if (dp.kv_group == 1) decode_split(B * H, Sk, dp.n_split, dp.chunk);
+  else decode_group_split(B * H, B * Hkv * cdiv(dp.kv_group, 16), Sk, dp.n_split, dp.chunk);
   dp.scale_log2 = float(double(scale) * 1.4426950408889634);
   dp.part = static_cast<float*>(workspace);
   dp.ml = dp.part + B * H * dp.n_split * D;

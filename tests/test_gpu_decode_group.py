@@ -1,0 +1,59 @@
+"""GPU parity of the grouped decode kernel (several query heads per kv head)
+at the sizes where it can go wrong: cache lengths around its 16-, 32- and
+128-key rounds and one split, groups below, at and above the 16 columns of a
+tile, head dims with idle V lanes, row strides, a running max that grows late.
+
+Bound: K.Q has exact products and fp32 sums, P and V are not rounded, so an
+fp32 output is within about S * 2^-24 of the weighted mean of |V|; 1e-5 holds
+that for S < 5000 and |V| < 5.  16-bit outputs add one rounding."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(dev, B, H, Hkv, S, D, dtype, k_pad=0, boost=None):
+    from minference.backend.attention import decode_dense
+
+    g = torch.Generator("cpu").manual_seed(S + D + H)
+    q = torch.randn(B, H, 1, D, generator=g).to(dtype)
+    k, v = (torch.randn(B, S, Hkv, D + k_pad, generator=g).to(dtype) for _ in range(2))
+    if boost:
+        for j, f in boost:
+            k[:, j] *= f
+    qd, kd, vd = (t.to(dev) for t in (q, k, v))
+    kv = [t[..., :D].transpose(1, 2) for t in (kd, vd)]
+    out = torch.empty(q.shape, dtype=torch.float32, device=dev)
+    decode_dense(qd, *kv, out=out)
+    o16 = decode_dense(qd, *kv)
+    qn = q.double().numpy()
+    kn, vn = (t[..., :D].transpose(1, 2).double().numpy().repeat(H // Hkv, axis=1) for t in (k, v))
+    x = (qn @ kn.swapaxes(-1, -2)) / np.sqrt(D)
+    p = np.exp(x - x.max(-1, keepdims=True))
+    ref = p @ vn / p.sum(-1, keepdims=True)
+    assert np.abs(out.cpu().double().numpy() - ref).max() < 1e-5
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    assert (np.abs(o16.cpu().double().numpy() - ref) <= 1e-5 + ulp * np.abs(ref)).all()
+
+
+@pytest.mark.parametrize("S", [1, 15, 16, 17, 31, 33, 64, 127, 128, 129, 500, 1025, 4113])
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (96, torch.float16),
+                                     (128, torch.bfloat16), (256, torch.float16)])
+def test_lengths(gpu_device, S, D, dtype):
+    _check(gpu_device, 2, 8, 2, S, D, dtype)
+
+
+@pytest.mark.parametrize("H,Hkv", [(2, 1), (6, 2), (15, 1), (16, 1), (17, 1), (40, 1), (64, 2)])
+def test_groups(gpu_device, H, Hkv):
+    _check(gpu_device, 1, H, Hkv, 333, 96, torch.bfloat16)
+    _check(gpu_device, 3, H, Hkv, 70, 512 if H < 10 else 128, torch.float16)
+
+
+def test_row_stride_and_late_maximum(gpu_device):
+    _check(gpu_device, 1, 4, 1, 900, 96, torch.bfloat16, k_pad=40)
+    _check(gpu_device, 1, 4, 2, 2000, 128, torch.bfloat16,
+           boost=[(3, 3.0), (700, 8.0), (1500, 30.0), (1999, 60.0)])
