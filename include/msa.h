@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MSA_ABI_VERSION 13
+#define MSA_ABI_VERSION 14
 
 /* status codes (negative: validation, nothing launched) */
 #define MSA_OK 0
@@ -353,6 +353,20 @@ int msa_decode_attention_noalloc(const msa_tensor4* q, const msa_tensor4* k,
 int msa_rope_qk(const msa_tensor4* q, const msa_tensor4* k, const msa_tensor4* cos,
                 const msa_tensor4* sin, const msa_tensor4* q_out, const msa_tensor4* k_out,
                 msa_stream_t stream);
+
+/* A caller's block ids as the lists msa_layer_attention takes (the set
+ * semantics of the reference's scatter into a block mask,
+ * minference/ops/block_sparse_kernel_npu.py:290-291): per 64-row query tile
+ * the distinct tiles ascending, repeats once, ids outside the key range
+ * dropped.  A block of 64 m tokens is its m consecutive tiles.
+ *   ids [pairs][rows_in][topk_in] int32 (ids64 = 0) or int64 (1), contiguous,
+ *       rows_in = ceil(s_q / block); any values
+ *   block: tokens per block, a multiple of 64
+ *   idx [pairs][n_qb][topk_in * m] int32: cnt tiles, then zeros
+ *   cnt [pairs][n_qb] int32; n_qb = ceil(s_q / 64) */
+int msa_block_lists(const void* ids, int32_t ids64, int64_t pairs, int64_t rows_in, int32_t topk_in,
+                    int32_t block, int64_t s_q, int64_t s_k, int32_t* idx, int32_t* cnt,
+                    msa_stream_t stream);
 
 /* Rounding of n (1..4) float32 tensors to fp16 (nearest even), one launch:
  * the inputs of ops called with float32 tensors (the reference's CPU paths

@@ -1018,6 +1018,31 @@ int msa_rope_qk(const msa_tensor4* q, const msa_tensor4* k, const msa_tensor4* c
   return e == hipSuccess ? MSA_OK : int(e);
 }
 
+int msa_block_lists(const void* ids, int32_t ids64, int64_t pairs, int64_t rows_in, int32_t topk_in,
+                    int32_t block, int64_t s_q, int64_t s_k, int32_t* idx, int32_t* cnt,
+                    msa_stream_t stream) {
+  if (!ids || !idx || !cnt) return MSA_E_NULL;
+  if (block < MSA_BLOCK || block % MSA_BLOCK != 0 || block > kMaxSeq) return MSA_E_BLOCK;
+  if (s_q < 1 || s_q > kMaxSeq || s_k < 1 || s_k > kMaxSeq) return MSA_E_SEQ;
+  const int m = block / MSA_BLOCK;
+  if (pairs < 1 || rows_in != cdiv(s_q, block)) return MSA_E_RANK;
+  if (topk_in < 1 || int64_t(topk_in) * m > 0x7fffffffLL) return MSA_E_TOPK;
+  ListParams lp;
+  lp.ids = ids;
+  lp.idx = idx;
+  lp.cnt = cnt;
+  lp.ids64 = ids64 != 0;
+  lp.rows_in = int(rows_in);
+  lp.topk_in = topk_in;
+  lp.m = m;
+  lp.n_qb = int(cdiv(s_q, MSA_BLOCK));
+  lp.n_kb = int(cdiv(s_k, MSA_BLOCK));
+  if (pairs > 0x7fffffffLL / lp.n_qb) return MSA_E_HEADS;
+  lp.pairs = int(pairs);
+  const hipError_t e = launch_block_lists(lp, reinterpret_cast<hipStream_t>(stream));
+  return e == hipSuccess ? MSA_OK : int(e);
+}
+
 int msa_round_f32(const msa_tensor4* src, const msa_tensor4* dst, int32_t n, int32_t* flag,
                   msa_stream_t stream) {
   if (!src || !dst || !flag) return MSA_E_NULL;

@@ -219,6 +219,19 @@ struct RopeParams {
   int batch, heads, kv_heads, s, rot, half, n_pair, n_pass;
 };
 
+// Block ids of a caller as the attention kernels' lists (block_lists_kernel).
+struct ListParams {
+  const void* ids;   // [pairs][rows_in][topk_in] int32 or int64
+  int32_t* idx;      // [pairs][n_qb][topk_in * m]
+  int32_t* cnt;      // [pairs][n_qb]
+  int ids64;         // 1: int64 ids
+  int pairs, rows_in, topk_in;
+  int m;             // tiles per block: id J names tiles m J .. m J + m - 1, row bq reads row bq / m
+  int n_qb, n_kb;    // 64-row query tiles, 64-key tiles
+};
+// Longest key axis of one list (its id bitmap lies in LDS).
+constexpr int kListMaxTiles = 16384;
+
 // float32 tensors rounded to fp16 in one launch (round_f16_kernel): source
 // strides in elements, contiguous fp16 outputs.
 constexpr int kRoundMax = 4;
@@ -252,6 +265,7 @@ hipError_t launch_attention_vs(const AttnParams& p, int dtype, int out_dtype, in
                                hipStream_t st);
 hipError_t launch_vs_build(const VsBuildParams& p, int n_bs, hipStream_t st);
 hipError_t launch_vs_estimate(const VsEstParams& p, int dtype, int D, hipStream_t st);
+hipError_t launch_block_lists(const ListParams& p, hipStream_t st);
 hipError_t launch_round(const RoundParams& p, int n, hipStream_t st);
 hipError_t launch_rope(const RopeParams& p, int dtype, hipStream_t st);
 

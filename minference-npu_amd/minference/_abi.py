@@ -53,7 +53,7 @@ MSA_ESTIMATE_SELECT_ONLY = 8
 
 MSA_MAX_HEADS = 128
 MSA_BLOCK = 64
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 _DTYPE_CODE = {
     torch.bfloat16: MSA_DTYPE_BF16,
@@ -82,6 +82,7 @@ EXPORTED_SYMBOLS = (
     "msa_vs_estimate",
     "msa_rope_qk",
     "msa_round_f32",
+    "msa_block_lists",
 )
 
 
@@ -247,6 +248,12 @@ def load_library() -> ctypes.CDLL:
         lib.msa_round_f32.argtypes = [
             ctypes.POINTER(MsaTensor4), ctypes.POINTER(MsaTensor4), ctypes.c_int32,
             ctypes.c_void_p, ctypes.c_void_p,
+        ]
+        lib.msa_block_lists.restype = ctypes.c_int
+        lib.msa_block_lists.argtypes = [
+            ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64, ctypes.c_int64, ctypes.c_int32,
+            ctypes.c_int32, ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p,
+            ctypes.c_void_p,
         ]
         ver = lib.msa_abi_version()
         if ver != ABI_VERSION:
@@ -419,6 +426,24 @@ def block_estimate(
             int(topk_max), float(score_scale), idx.data_ptr(), cnt.data_ptr(), ws.data_ptr(),
             ws.numel(), stream)
     check(st)
+
+
+def block_lists(ids: torch.Tensor, block: int, s_q: int, s_k: int):
+    """Launch msa_block_lists on the current stream: block ids [B, H,
+    n_q_blocks, topk] (int32 or int64, contiguous) of ``block``-token blocks
+    as the attention kernels' lists (idx [B, H, n_qb, topk * m], cnt [B, H,
+    n_qb]), int32, in 64-token tiles."""
+    B, H, rows, topk = ids.shape
+    if ids.dtype not in (torch.int32, torch.int64) or not ids.is_contiguous():
+        raise ValueError("block ids must be contiguous int32 or int64")
+    n_qb = -(-s_q // MSA_BLOCK)
+    idx = torch.empty((B, H, n_qb, topk * (int(block) // MSA_BLOCK)), dtype=torch.int32,
+                      device=ids.device)
+    cnt = torch.empty((B, H, n_qb), dtype=torch.int32, device=ids.device)
+    check(load_library().msa_block_lists(
+        ids.data_ptr(), int(ids.dtype == torch.int64), B * H, rows, topk, int(block), s_q, s_k,
+        idx.data_ptr(), cnt.data_ptr(), current_stream_handle(ids.device)))
+    return idx, cnt
 
 
 def head_descs(heads: Sequence[tuple]):

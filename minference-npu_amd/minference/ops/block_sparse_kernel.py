@@ -141,21 +141,25 @@ def block_sparse_attention_with_indices(
             "block_indices shape must be [B,H,n_q_blocks,topk_blocks]; "
             f"got {tuple(block_indices.shape)} for q={tuple(q.shape)} block_size={block_size}"
         )
-    ids = block_indices.to(q.device)
-    if bs != _abi.MSA_BLOCK:
-        ids = tile_ids(ids, bs, math.ceil(S_q / _abi.MSA_BLOCK))
-    n_kb = math.ceil(k.shape[2] / _abi.MSA_BLOCK)
-    idx, cnt = canonical_block_lists(ids, n_kb)
+    return _attend_ids(q, k, v, block_indices.to(q.device), bs, out)
+
+
+def _attend_ids(q, k, v, ids, bs, out):
+    """Attention over the ids [B, H, n_q_blocks, topk] (q's device) of
+    ``bs``-token blocks: one launch turns them into the kernel's tile lists."""
+    if ids.dtype not in (torch.int32, torch.int64):
+        ids = ids.long()
+    idx, cnt = _abi.block_lists(ids.contiguous(), bs, q.shape[2], k.shape[2])
     topk = idx.shape[-1]
     chunks = []
-    for h0, h1 in head_chunks(H):
+    for h0, h1 in head_chunks(q.shape[1]):
         chunks.append((h0, h1, idx[:, h0:h1].contiguous(), cnt[:, h0:h1].contiguous()))
     scale = sparse_scale(q.shape[-1])
     return padded_call(q, k, v, out, lambda q, k, v, r: _run(q, k, v, chunks, topk, scale, r))
 
 
 def tile_ids(block_indices: torch.Tensor, block_size: int, n_qb: int) -> torch.Tensor:
-    """Ids of ``block_size``-token blocks [B, H, n_q_blocks, topk] as ids of
+    """The first half of msa_block_lists in torch ops (any device): ids of ``block_size``-token blocks [B, H, n_q_blocks, topk] as ids of
     the kernels' 64-token tiles [B, H, n_qb, topk * m] (m = block_size / 64):
     block J is tiles m J .. m J + m - 1, and 64-row query block bq takes the
     list of its block bq // m.  The token visibility is unchanged: a key is
@@ -169,8 +173,8 @@ def tile_ids(block_indices: torch.Tensor, block_size: int, n_qb: int) -> torch.T
 
 
 def canonical_block_lists(block_indices: torch.Tensor, n_kb: int):
-    """Turn arbitrary per-row block ids into the kernel's list format: the
-    distinct ids in [0, n_kb) ascending first, ``cnt`` = how many.  This is the
+    """The second half of msa_block_lists in torch ops (any device): turn
+    arbitrary per-row block ids into the kernel's list format: the distinct ids in [0, n_kb) ascending first, ``cnt`` = how many.  This is the
     set semantics of the reference's scatter into a block mask
     (block_sparse_kernel_npu.py:290-291): repeats count once and ids outside
     the key range select nothing.  Returns int32 (idx, cnt)."""
@@ -229,14 +233,16 @@ def block_sparse_attention(
     check_bnsd(q, k, v)
     check_supported(q, k, v)
     _check_block_size(block_size)
-    if int(block_size) != _abi.MSA_BLOCK:
-        ids = select_block_sparse_topk_indices(q, k, topk_blocks, block_size,
-                                               force_first=force_first, force_diag=force_diag)
-        return block_sparse_attention_with_indices(q, k, v, ids, block_size, out=out)
-    n_kb = math.ceil(k.shape[2] / _abi.MSA_BLOCK)
+    bs = int(block_size)
+    n_kb = math.ceil(k.shape[2] / bs)
     topk = min(max(1, int(topk_blocks)), n_kb)
     scale = sparse_scale(q.shape[-1])
     flags = select_flags(force_first, force_diag)
+    if bs != _abi.MSA_BLOCK:
+        dk = kernel_head_dim(q.shape[-1])
+        ids = [c[2] for c in _estimate(kernel_view(pad_head_dim(q, dk)),
+                                       kernel_view(pad_head_dim(k, dk)), topk, scale, flags, bs)]
+        return _attend_ids(q, k, v, ids[0] if len(ids) == 1 else torch.cat(ids, dim=1), bs, out)
 
     def run(q, k, v, result):
         _run(q, k, v, _estimate(q, k, topk, scale, flags), topk, scale, result)
