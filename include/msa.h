@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define MSA_ABI_VERSION 14
+#define MSA_ABI_VERSION 15
 
 /* status codes (negative: validation, nothing launched) */
 #define MSA_OK 0
@@ -213,6 +213,24 @@ int msa_layer_attention_staged(const msa_tensor4* q, const msa_tensor4* k,
                                const int32_t* idx, const int32_t* cnt,
                                int32_t idx_slots, int32_t topk_max, void* workspace,
                                size_t workspace_bytes, msa_stream_t stream);
+
+/* msa_layer_attention (stage = 1) or msa_layer_attention_staged (stage = 0)
+ * with room to split long items over their keys: one workgroup walks the keys
+ * of one (head, 64-row query block), so a few query blocks against a long key
+ * axis (a chunk of a prompt) leave most of the GPU idle.  With a split
+ * workspace such items are cut into key splits and merged by one more launch;
+ * msa_split_workspace_bytes says how much this call would use (0: nothing is
+ * split, split_workspace may be NULL, which always means no splits).  Same
+ * results up to the rounding of the last fp32 sums.  vertical_and_slash heads
+ * go through msa_layer_attention_ex.  Same reference counterpart as msa_layer_attention. */
+size_t msa_split_workspace_bytes(const msa_tensor4* q, const msa_tensor4* k,
+                                 const msa_head_desc* heads, int32_t n_heads, int32_t topk_max);
+int msa_layer_attention_split(const msa_tensor4* q, const msa_tensor4* k, const msa_tensor4* v,
+                              const msa_tensor4* o, const msa_head_desc* heads, int32_t n_heads,
+                              const int32_t* idx, const int32_t* cnt, int32_t idx_slots,
+                              int32_t topk_max, void* split_workspace,
+                              size_t split_workspace_bytes, void* workspace,
+                              size_t workspace_bytes, int32_t stage, msa_stream_t stream);
 
 /* msa_stage_kv and the pooling pass of the block estimator in one launch, for
  * the layer schedule of a layer with block_sparse heads:

@@ -281,6 +281,11 @@ static int* queue_of(void* workspace, size_t workspace_bytes) {
                                 kQueueBytes);
 }
 
+// flag of the staging behind the counters: K read in place or staged
+static int32_t* k_flag_of(void* workspace, size_t workspace_bytes) {
+  return queue_of(workspace, workspace_bytes) + 16;
+}
+
 // CUs per XCD of the current device (8 XCDs on gfx950)
 static int cus_per_xcd() {
   int dev = 0, cus = 256;
@@ -305,14 +310,36 @@ static int cus_per_xcd() {
 // us in place and 2270 us staged (8000 tokens: 1081 and 1002); contiguous
 // rows of 96 (64K headline layer) 4.51 ms in place, 4.54 staged.  D = 512
 // always takes staged K: its kernel reads every tile's K once per wave.
-static bool k_in_place(const msa_tensor4* k) {
+static bool k_can_stay(const msa_tensor4* k) {
   const int64_t D = k->size[3], ss = k->stride[2];
   const int64_t s_pad = cdiv(k->size[2], MSA_BLOCK) * MSA_BLOCK;
-  return D <= 256 && ss % 64 == 32 && ss >= D && (s_pad * ss + D) * 2 <= (int64_t(1) << 31);
+  return D <= 256 && ss >= D && (s_pad * ss + D) * 2 <= (int64_t(1) << 31);
+}
+static bool k_stride_slow(const msa_tensor4* k) { return k->stride[2] % 64 != 32; }
+// what msa_stage_kv and every full prefill (S_q == S_k) leave in place
+static bool k_in_place(const msa_tensor4* k) { return k_can_stay(k) && !k_stride_slow(k); }
+
+// Staging K pays where enough query blocks read it: with few (a chunk of a
+// prompt against a long cache) the copy costs more than the loads it speeds
+// up.  A K tile's copy takes about 6.5 ns of the GPU at D = 128, a staged
+// tile's loads save about 60 ns of one CU: 27 uses.  The line is drawn at 32
+// (query blocks x query heads per kv head), for S_q < S_k only: in a full
+// prefill of that size K is a few MB.  (2000 rows of 30000 keys, 32 heads on
+// 8 x 128, 128 uses at most: whole layer 476 us staged, 489 in place.)
+static bool k_used_enough(const msa_tensor4* q, const msa_tensor4* k) {
+  return q->size[2] == k->size[2] ||
+         cdiv(q->size[2], MSA_BLOCK) * (q->size[1] / k->size[1]) >= 32;
 }
 
-static int stage_setup(const msa_tensor4* k, const msa_tensor4* v, void* workspace,
-                       size_t workspace_bytes, StageParams& sp) {
+// q: the query tensor where the caller has it (null: K staged by its stride
+// alone).  The choice travels to the attention launch in the workspace.
+static int stage_k_mode(const msa_tensor4* q, const msa_tensor4* k) {
+  if (!k_can_stay(k)) return 1;
+  return k_stride_slow(k) && (!q || k_used_enough(q, k)) ? 1 : 0;
+}
+
+static int stage_setup(const msa_tensor4* q, const msa_tensor4* k, const msa_tensor4* v,
+                       void* workspace, size_t workspace_bytes, StageParams& sp) {
   if (!k || !v || !k->data || !v->data) return MSA_E_NULL;
   for (int i = 0; i < 4; ++i) {
     if (v->size[i] <= 0) return MSA_E_RANK;
@@ -343,7 +370,8 @@ static int stage_setup(const msa_tensor4* k, const msa_tensor4* v, void* workspa
   sp.kv_heads = int(Hkv);
   sp.s_k = int(Sk);
   sp.s_pad = int(cdiv(Sk, MSA_BLOCK) * MSA_BLOCK);
-  sp.stage_k = k_in_place(k) ? 0 : 1;
+  sp.stage_k = stage_k_mode(q, k);
+  sp.k_flag = k_flag_of(workspace, need);
   return MSA_OK;
 }
 
@@ -356,7 +384,7 @@ static int stage_launch(const StageParams& sp, int dtype, int D, hipStream_t hs)
 int msa_stage_kv(const msa_tensor4* k, const msa_tensor4* v, void* workspace,
                  size_t workspace_bytes, msa_stream_t stream) {
   StageParams sp;
-  const int st = stage_setup(k, v, workspace, workspace_bytes, sp);
+  const int st = stage_setup(nullptr, k, v, workspace, workspace_bytes, sp);
   if (st != MSA_OK) return st;
   return stage_launch(sp, v->dtype, int(v->size[3]), reinterpret_cast<hipStream_t>(stream));
 }
@@ -366,7 +394,7 @@ int msa_stage_kv_pool(const msa_tensor4* q, const msa_tensor4* k, const msa_tens
                       size_t est_workspace_bytes, void* workspace, size_t workspace_bytes,
                       msa_stream_t stream) {
   StageParams sp;
-  int st = stage_setup(k, v, workspace, workspace_bytes, sp);
+  int st = stage_setup(nullptr, k, v, workspace, workspace_bytes, sp);
   if (st != MSA_OK) return st;
   if (n_slots > 0) {
     int16_t slot_kvp[kMaxHeads];
@@ -375,6 +403,7 @@ int msa_stage_kv_pool(const msa_tensor4* q, const msa_tensor4* k, const msa_tens
                     slot_kvp, L);
     if (st != MSA_OK) return st;
     sp.n_pool_wg = pool_workgroups(sp.pool);
+    sp.stage_k = stage_k_mode(q, k);
   } else if (n_slots < 0) {
     return MSA_E_HEADS;
   }
@@ -504,17 +533,21 @@ size_t msa_vs_workspace_bytes(int64_t batch, int32_t n_slots, int64_t s_k, int32
   return vs_layout(batch, n_slots, s_k, v_stride, head_dim).total;
 }
 
-// Work model of one head for the XCD split: query block bq costs
-// min(bq + 1, cap) + fixed, in key tiles (fixed covers the item set-up and
-// the output merge).  The prefix sums have a closed form.
+// Work model of one head (or key split of one) for the XCD ranges: query
+// block bq costs min(bq + 1 + off, cap) key tiles, divided by the splits,
+// plus fixed (the item set-up and the output merge).  The prefix sums have a
+// closed form.
 struct HeadWork {
   double cap, fixed;
-  bool flat;  // every query block costs cap (no causal triangle)
+  double off;   // tiles before the first query block (S_q < S_k)
+  double div;   // key splits
+  bool flat;    // every query block costs cap (no causal triangle)
+  double longest(int n_qb) const { return flat ? cap : fmin(double(n_qb) + off, cap); }
 };
 
-static HeadWork head_work(const msa_head_desc& hd, int n_kb, int topk_max) {
+static HeadWork head_work(const msa_head_desc& hd, int n_qb, int n_kb, int topk_max) {
   const double nb = double(n_kb);
-  HeadWork w{nb, 2.0, hd.kind == MSA_KIND_FULL};
+  HeadWork w{nb, 2.0, fmax(double(n_kb - n_qb), 0.0), 1.0, hd.kind == MSA_KIND_FULL};
   if (hd.kind == MSA_KIND_STREAM) {
     w.cap = fmin(nb, double(hd.p2) / 64.0 + 2.0 + ceil(fmax(double(hd.p1), 0.0) / 64.0));
   } else if (hd.kind == MSA_KIND_BLOCK) {
@@ -529,22 +562,28 @@ static HeadWork head_work(const msa_head_desc& hd, int n_kb, int topk_max) {
 
 // cost of query blocks 0 .. m-1
 static double prefix_cost(const HeadWork& w, double m) {
-  const double k = w.cap;
-  if (w.flat) return m * (k + w.fixed);
-  const double tri = m <= k ? m * (m + 1) / 2 : k * (k + 1) / 2 + (m - k) * k;
-  return tri + w.fixed * m;
+  const double k = w.cap, a = w.off;
+  double tiles;
+  if (w.flat || k <= a) {
+    tiles = m * k;
+  } else {
+    const double up = fmin(m, k - a);  // blocks before the cap is reached
+    tiles = up * a + up * (up + 1) / 2 + (m - up) * k;
+  }
+  return tiles / w.div + w.fixed * m;
 }
 
-// Items of one launch: the listed (batch, head) pairs, head-major, query
-// blocks longest-first; the 8 XCDs (round-robin workgroup dispatch) take
-// contiguous ranges of equal estimated cost, so each XCD's L2 serves few
-// heads and a heavy head can be shared by two XCDs.
-static void order_items(AttnParams& ap, const int* pairs, const HeadWork* work, int n) {
+// Items of one launch: the listed entries ((batch, head) pairs or key splits
+// of one, AttnParams::head_order codes), head-major, query blocks
+// longest-first; the 8 XCDs (round-robin workgroup dispatch) take contiguous
+// ranges of equal estimated cost, so each XCD's L2 serves few heads and a
+// heavy head can be shared by two XCDs.
+static void order_items(AttnParams& ap, const int* entries, const HeadWork* work, int n) {
   const int nq = ap.n_qb;
   ap.n_hl = n;
-  double head_tot[kMaxHeads], total = 0.0;
+  double head_tot[kMaxEntries], total = 0.0;
   for (int i = 0; i < n; ++i) {
-    ap.head_order[i] = pairs[i];
+    ap.head_order[i] = entries[i];
     head_tot[i] = prefix_cost(work[i], nq);
     total += head_tot[i];
   }
@@ -587,12 +626,95 @@ static void interleave_kinds(int* list, int n, const msa_head_desc* heads, int H
   }
 }
 
+// Item list of a launch without vertical_and_slash heads: every (batch, head)
+// pair but the skipped ones, and the key splits.
+struct ItemPlan {
+  int n = 0;                 // entries
+  int n_split = 1, n_sp = 0;  // splits per split pair, split pairs
+  int entry[kMaxEntries];
+  HeadWork work[kMaxEntries];
+  uint8_t pair[kMaxHeads];   // of each split pair
+  // floats of the partial outputs
+  size_t part_floats(int n_qb, int D) const {
+    return size_t(n_sp) * n_split * n_qb * MSA_BLOCK * (size_t(D) + 2);
+  }
+};
+
+// Key splits: an item is one workgroup, so a launch takes at least as long as
+// its longest item.  Where that is well above the average load of the
+// workgroups the GPU holds at once (a chunk of a prompt against a long cache),
+// the long heads are cut into up to kMaxSplit key splits whose partial outputs
+// a second launch merges.  The piece aimed at is half the average load, and
+// not below 64 tiles; heads below 160 tiles stay whole: a piece writes 25 to
+// 64 KB that the merge (5 to 8 us) reads again, more than shorter heads gain
+// (4 dense heads x 6000 x 96, 94 tiles: 50 us whole, 59 in pieces of 24).  At
+// D >= 128 a tile takes about twice as long, so the lines lie at 32 and 96
+// (300 rows of 20000 keys, 32 heads on 8 x 128, 100 tiles: 101 us whole, 93
+// in pieces of 32; D = 64: 83.4 whole, 84.8).
+// 2000 rows of 30000 keys, 32 heads, 30 % stream / 60 % block / 10 % dense,
+// whole layer: D = 96 407 -> 320 us, D = 128 476 -> 363 us; 100 rows of 40000
+// keys: 427 -> 193 us.
+static void plan_items(const msa_head_desc* heads, int H, int BH, int n_qb, int n_kb, int topk_max,
+                       int D, bool split, ItemPlan& pl) {
+  int pairs[kMaxHeads];
+  HeadWork work[kMaxHeads];
+  int n = 0;
+  for (int i = 0; i < BH; ++i)
+    if (heads[i % H].kind != MSA_KIND_SKIP && heads[i % H].kind != MSA_KIND_VS) pairs[n++] = i;
+  interleave_kinds(pairs, n, heads, H);
+  double total = 0.0, longest = 0.0;
+  for (int i = 0; i < n; ++i) {
+    work[i] = head_work(heads[pairs[i] % H], n_qb, n_kb, topk_max);
+    total += prefix_cost(work[i], n_qb);
+    longest = fmax(longest, work[i].longest(n_qb));
+  }
+  const double slots = 8.0 * cus_per_xcd() * (D > 128 ? 1 : 2);
+  const double piece = fmax(total / slots / 2.0, D < 128 ? 64.0 : 32.0);
+  const double least = fmax(D < 128 ? 160.0 : 96.0, 1.5 * piece);
+  int ns = 1, n_sp = 0;
+  if (split && D <= 256 && longest > least) {
+    ns = int(fmin(double(kMaxSplit), ceil(longest / piece)));
+    for (int i = 0; i < n; ++i) n_sp += work[i].longest(n_qb) > least;
+    while (ns > 1 && n + (ns - 1) * n_sp > kMaxEntries) --ns;
+  }
+  pl.n = 0;
+  pl.n_sp = 0;
+  pl.n_split = ns;
+  for (int i = 0; i < n; ++i) {
+    if (ns == 1 || work[i].longest(n_qb) <= least) {
+      pl.entry[pl.n] = pairs[i];
+      pl.work[pl.n++] = work[i];
+      continue;
+    }
+    work[i].div = ns;
+    for (int k = 0; k < ns; ++k) {
+      pl.entry[pl.n] = int(0x80000000u | uint32_t(k) << 16 | uint32_t(pl.n_sp) << 8 | uint32_t(pairs[i]));
+      pl.work[pl.n++] = work[i];
+    }
+    pl.pair[pl.n_sp++] = uint8_t(pairs[i]);
+  }
+}
+
+size_t msa_split_workspace_bytes(const msa_tensor4* q, const msa_tensor4* k,
+                                 const msa_head_desc* heads, int32_t n_heads, int32_t topk_max) {
+  if (check_qk(q, k) != MSA_OK || !heads || n_heads != q->size[1] || n_heads > kMaxHeads) return 0;
+  const int64_t BH = q->size[0] * q->size[1];
+  if (BH > kMaxHeads) return 0;
+  for (int h = 0; h < n_heads; ++h)
+    if (heads[h].kind == MSA_KIND_VS) return 0;
+  const int n_qb = int(cdiv(q->size[2], MSA_BLOCK)), n_kb = int(cdiv(k->size[2], MSA_BLOCK));
+  ItemPlan pl;
+  plan_items(heads, n_heads, int(BH), n_qb, n_kb, topk_max, int(q->size[3]), true, pl);
+  return pl.part_floats(n_qb, int(q->size[3])) * 4;
+}
+
 static int layer_attention_impl(const msa_tensor4* q, const msa_tensor4* k, const msa_tensor4* v,
                                 const msa_tensor4* o, const msa_head_desc* heads, int32_t n_heads,
                                 const int32_t* idx, const int32_t* cnt, int32_t idx_slots,
                                 int32_t topk_max, const msa_vs_lists* vs, void* vs_workspace,
                                 size_t vs_workspace_bytes, void* workspace,
-                                size_t workspace_bytes, msa_stream_t stream, bool stage) {
+                                size_t workspace_bytes, msa_stream_t stream, bool stage,
+                                void* split_ws = nullptr, size_t split_ws_bytes = 0) {
   int st = check_qk(q, k);
   if (st != MSA_OK) return st;
   if (!v || !o || !v->data || !o->data || !heads) return MSA_E_NULL;
@@ -659,11 +781,18 @@ static int layer_attention_impl(const msa_tensor4* q, const msa_tensor4* k, cons
   if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return MSA_E_ALIGN;
   if (int64_t(n_qb) * B * H > 0x7fffffffLL) return MSA_E_SEQ;
   if (B * Hkv > 65535) return MSA_E_HEADS;
+  const int BH = int(B * H);
+  ItemPlan pl;
+  if (n_vs == 0 && BH <= kMaxHeads) {
+    plan_items(heads, int(H), BH, n_qb, n_kb, topk_max, D, split_ws != nullptr, pl);
+    if (pl.n_sp && split_ws_bytes < pl.part_floats(n_qb, D) * 4) return MSA_E_WORKSPACE;
+    if (pl.n_sp && (reinterpret_cast<uintptr_t>(split_ws) & 255u) != 0) return MSA_E_ALIGN;
+  }
 
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
   if (stage) {
     StageParams sp;
-    st = stage_setup(k, v, workspace, workspace_bytes, sp);
+    st = stage_setup(q, k, v, workspace, workspace_bytes, sp);
     if (st == MSA_OK) st = stage_launch(sp, v->dtype, D, hs);
     if (st != MSA_OK) return st;
   }
@@ -675,7 +804,7 @@ static int layer_attention_impl(const msa_tensor4* q, const msa_tensor4* k, cons
   const AttnLayout AL = attn_layout(B, Hkv, Sk, D);
   ap.vt = ws_at<uint16_t>(workspace, AL.vt);
   ap.kt = ws_at<uint16_t>(workspace, AL.kt);
-  ap.k_in_place = k_in_place(k) ? 1 : 0;
+  ap.k_flag = k_flag_of(workspace, need);
   int32_t* vexp = ws_at<int32_t>(workspace, AL.vexp);
   ap.vexp = vexp;
   ap.o = o->data;
@@ -706,22 +835,30 @@ static int layer_attention_impl(const msa_tensor4* q, const msa_tensor4* k, cons
     ap.hd[h].scale_log2 = float(double(heads[h].scale) * log2e);
   }
 
-  const int BH = int(B * H);
   if (n_vs == 0) {
     if (BH <= kMaxHeads) {
-      int pairs[kMaxHeads];
-      HeadWork work[kMaxHeads];
-      int n = 0;
-      for (int i = 0; i < BH; ++i)
-        if (heads[i % H].kind != MSA_KIND_SKIP) pairs[n++] = i;
-      if (n == 0) return MSA_OK;
-      interleave_kinds(pairs, n, heads, int(H));
-      for (int i = 0; i < n; ++i) work[i] = head_work(heads[pairs[i] % H], n_kb, topk_max);
-      order_items(ap, pairs, work, n);
+      if (pl.n == 0) return MSA_OK;
+      order_items(ap, pl.entry, pl.work, pl.n);
+      ap.n_split = pl.n_split;
+      ap.part = static_cast<float*>(split_ws);
     } else {
       ap.n_hl = 0;  // every pair, plain order
     }
-    const hipError_t e = launch_attention(ap, q->dtype, o->dtype, D, hs);
+    hipError_t e = launch_attention(ap, q->dtype, o->dtype, D, hs);
+    if (e == hipSuccess && BH <= kMaxHeads && pl.n_sp) {
+      CombineParams cp;
+      memset(&cp, 0, sizeof(cp));
+      cp.part = ap.part;
+      cp.o = ap.o;
+      cp.o_sb = ap.o_sb; cp.o_sh = ap.o_sh; cp.o_ss = ap.o_ss;
+      cp.heads = ap.heads;
+      cp.s_q = ap.s_q;
+      cp.n_qb = n_qb;
+      cp.n_split = pl.n_split;
+      cp.n_pairs = pl.n_sp;
+      memcpy(cp.pair, pl.pair, sizeof(cp.pair));
+      e = launch_combine(cp, q->dtype, o->dtype, D, hs);
+    }
     return e == hipSuccess ? MSA_OK : int(e);
   }
 
@@ -772,25 +909,25 @@ static int layer_attention_impl(const msa_tensor4* q, const msa_tensor4* k, cons
     const msa_head_desc& hd = heads[i % H];
     if (hd.kind == MSA_KIND_VS) {
       vs_pairs[n_v] = i;
-      vs_work[n_v++] = head_work(hd, n_kb, topk_max);
+      vs_work[n_v++] = head_work(hd, n_qb, n_kb, topk_max);
     } else if (hd.kind != MSA_KIND_SKIP) {
       other[n_o++] = i;
     }
   }
   interleave_kinds(other, n_o, heads, int(H));
-  for (int i = 0; i < n_o; ++i) other_work[i] = head_work(heads[other[i] % H], n_kb, topk_max);
-  if (ap.k_in_place) {
+  for (int i = 0; i < n_o; ++i) other_work[i] = head_work(heads[other[i] % H], n_qb, n_kb, topk_max);
+  if (k_in_place(k)) {
     // the vertical_and_slash kernel reads staged K: stage the K the plain
     // staging left in place (V and its exponents are staged already)
     StageParams kp;
-    st = stage_setup(k, v, workspace, workspace_bytes, kp);
+    st = stage_setup(nullptr, k, v, workspace, workspace_bytes, kp);
     if (st != MSA_OK) return st;
     kp.stage_k = 2;
+    kp.k_flag = nullptr;  // the other heads' launch still reads K in place
     e = launch_stage(kp, q->dtype, D, hs);
     if (e != hipSuccess) return int(e);
   }
   AttnParams vp = ap;
-  vp.k_in_place = 0;
   vp.vs_lists = bp.lists;
   vp.vs_cnt = bp.cnt;
   vp.gkt = gp.kt;
@@ -824,6 +961,17 @@ int msa_layer_attention_staged(const msa_tensor4* q, const msa_tensor4* k, const
                                msa_stream_t stream) {
   return layer_attention_impl(q, k, v, o, heads, n_heads, idx, cnt, idx_slots, topk_max,
                               nullptr, nullptr, 0, workspace, workspace_bytes, stream, false);
+}
+
+int msa_layer_attention_split(const msa_tensor4* q, const msa_tensor4* k, const msa_tensor4* v,
+                              const msa_tensor4* o, const msa_head_desc* heads, int32_t n_heads,
+                              const int32_t* idx, const int32_t* cnt, int32_t idx_slots,
+                              int32_t topk_max, void* split_workspace,
+                              size_t split_workspace_bytes, void* workspace,
+                              size_t workspace_bytes, int32_t stage, msa_stream_t stream) {
+  return layer_attention_impl(q, k, v, o, heads, n_heads, idx, cnt, idx_slots, topk_max, nullptr,
+                              nullptr, 0, workspace, workspace_bytes, stream, stage != 0,
+                              split_workspace, split_workspace_bytes);
 }
 
 int msa_layer_attention_ex(const msa_tensor4* q, const msa_tensor4* k, const msa_tensor4* v,

@@ -203,6 +203,8 @@ __global__ __launch_bounds__(256) void stage_kernel(StageParams P) {
     b = bk / P.kv_heads;
     kvh = bk - b * P.kv_heads;
   }
+  // for the attention launch: whether it finds K in its own rows
+  if (wi == 0 && P.k_flag && threadIdx.x == 0) *P.k_flag = P.stage_k == 0 ? 1 : 0;
   // the tile's 4 chunks are 64*D consecutive halves starting at key j0
   const int64_t dst0 = (int64_t(bk) * P.s_pad + j0) * D;
   if (plane == 1) {
@@ -398,6 +400,13 @@ struct TileSeq {
     total = c;
     mpos = nfull == 1 ? c1 : c2;
   }
+  // Keep positions [at, end) only, renumbered from 0.
+  __device__ void narrow(int at, int end) {
+    lo0 += at;
+    c1 -= at; c2 -= at; c3 -= at; c4 -= at;
+    mpos -= at;
+    total = end - at;
+  }
   // Tile at position q, clamped into [0, n_kb) for memory safety; positions
   // past the end repeat the last tile (loads that are never consumed).  In
   // two halves, so that a caller can issue the scalar load a step before it
@@ -463,6 +472,49 @@ __device__ inline void item_tiles(const AttnParams& P, int kind, int64_t list_ro
   } else {
     seq.set({0, Fe, 0, 0, 0}, {Fe, last_tile + 1, 0, 0, 0}, 1);
   }
+}
+
+// An item of the list: its (batch, head) pair and query block, and for a key
+// split its share of the tiles and its place in the partial outputs.
+struct Item {
+  int hh, bq;
+  int split;     // -1: the whole item
+  int part_row;  // row of AttnParams::part
+};
+
+// Workgroup i's item of a launch of one item each; false: none.
+__device__ inline bool find_item(const AttnParams& P, Item& it) {
+  const int xcd = blockIdx.x & 7;
+  it.split = -1;
+  it.part_row = 0;
+  if (P.n_hl) {
+    const int r = int(blockIdx.x) >> 3;
+    if (r >= P.xcd_count[xcd]) return false;
+    const int g = P.xcd_start[xcd] + r;
+    const int hl = g / P.n_qb;
+    const int e = P.head_order[hl];
+    it.hh = e & 0xff;
+    it.bq = P.n_qb - 1 - (g - hl * P.n_qb);
+    if (e < 0) {
+      it.split = (e >> 16) & 0xff;
+      it.part_row = (((e >> 8) & 0xff) * P.n_split + it.split) * P.n_qb + it.bq;
+    }
+  } else {
+    // plain order: every (batch, head) pair; the host lists no item of a
+    // skipped head in the other mode
+    const int BH = P.batch * P.heads;
+    it.hh = int(blockIdx.x) % BH;
+    if (P.hd[it.hh % P.heads].kind == KIND_SKIP) return false;
+    it.bq = P.n_qb - 1 - int(blockIdx.x) / BH;
+  }
+  return true;
+}
+
+// Partial output of a key split: 64 x D floats (each row normalised by its
+// own sum), then (m, l) of the 64 rows.
+template <int D>
+__device__ inline float* part_of(const AttnParams& P, int row) {
+  return P.part + int64_t(row) * (kBlock * (D + 2));
 }
 
 template <typename TO>
@@ -540,6 +592,9 @@ void attn_kernel(AttnParams P) {
   __shared__ int s_item;
   const int xcd = blockIdx.x & 7;
 
+  bool k_in_place = false;
+  if constexpr (!VS) k_in_place = load_uniform(P.k_flag) != 0;
+
   // ---- state of the current work item (wave-uniform)
   int b = 0, h = 0, q0 = 0, a0 = 0, n_init = 0, n_local = 0, kind = KIND_DENSE;
   float c_log2 = 0.0f, vfac = 1.0f;
@@ -552,7 +607,7 @@ void attn_kernel(AttnParams P) {
   bool is_full = false, is_stream = false;
   const int skm1 = P.s_k - 1;
 
-  auto init_item = [&](const int hh, const int bq) INLINE {
+  auto init_item = [&](const int hh, const int bq, const int split) INLINE {
     b = hh / P.heads;
     h = hh - b * P.heads;
     const int kvh = h / P.kv_group;
@@ -578,14 +633,16 @@ void attn_kernel(AttnParams P) {
     } else {
       item_tiles(P, kind, (int64_t(b) * P.idx_slots + hd_slot) * P.n_qb + bq, a0, a1, n_init,
                  n_local, seq);
+      if (split >= 0)
+        seq.narrow(seq.total * split / P.n_split, seq.total * (split + 1) / P.n_split);
     }
     total = seq.total;
-    mpos = min(seq.mpos, total);
+    mpos = max(min(seq.mpos, total), 0);
 
     const int64_t bk = int64_t(b) * (P.heads / P.kv_group) + kvh;
     // staged V is V * 2^-vexp (stage_kernel); the output takes the 2^vexp back
     vfac = __builtin_amdgcn_ldexpf(1.0f, load_uniform(P.vexp + bk));
-    if (!VS && P.k_in_place) {
+    if (k_in_place) {
       // the head's own K rows; the record count ends at the last row's last
       // element, so rows past S_k (and dropped loads) read zeros
       krs = __builtin_amdgcn_make_buffer_rsrc(
@@ -665,7 +722,6 @@ void attn_kernel(AttnParams P) {
   // load returns zeros without a memory access (the loop's instruction
   // stream stays the same).
   const uint32_t lane_off = 16u * lane;
-  const bool k_in_place = !VS && P.k_in_place;
   const uint32_t k_row_bytes = uint32_t(P.k_ss) * 2u;
   const uint32_t k_lane = k_in_place ? uint32_t(lc) * k_row_bytes + 16u * lr : lane_off;
   const uint32_t k_cv = k_in_place ? 16u * k_row_bytes : 0u;  // VGPR bytes per chunk
@@ -927,7 +983,9 @@ void attn_kernel(AttnParams P) {
   // hold group 2rb+1, chosen by an exact blend (the maxima are finite)
   // rather than a select, which the compiler turns into a lane-indexed load
   // from a private copy of m_g.
-  auto merge_store = [&](const int ib, const int ih, const int iq0, const float iv) INLINE {
+  // A key split leaves them, with its rows' (m, l), in the partial outputs.
+  auto merge_store = [&](const int ib, const int ih, const int iq0, const float iv,
+                         float* const pdst) INLINE {
     float m_b[2], l_b[2];
     const float odd = float(lr & 1);
 #pragma unroll
@@ -978,6 +1036,8 @@ void attn_kernel(AttnParams P) {
         for (int c = 0; c < 4; ++c) f[c] *= inv;
 
         const int row = iq0 + 32 * rb + (lane & 31);
+        if (!VS && pdst && W == 0 && lane < 32)
+          *reinterpret_cast<float2*>(pdst + kBlock * D + 2 * (row - iq0)) = make_float2(mt, lt);
         if (row < P.s_q) {
           const int64_t obase = ib * P.o_sb + int64_t(ih) * P.o_sh + int64_t(row) * P.o_ss;
 #pragma unroll
@@ -1003,7 +1063,9 @@ void attn_kernel(AttnParams P) {
               v4[3] = __builtin_fmaf(pc[c].w, f[c], v4[3]);
             }
             const int d = 32 * db + 8 * W + 4 * (lane >> 5);
-            if constexpr (OUT_F32) {
+            if (!VS && pdst) {
+              store_out4<float>(pdst + (row - iq0) * D + d, v4[0], v4[1], v4[2], v4[3]);
+            } else if constexpr (OUT_F32) {
               store_out4<float>(reinterpret_cast<float*>(P.o) + obase + d, v4[0], v4[1], v4[2],
                                 v4[3]);
             } else {
@@ -1028,36 +1090,22 @@ void attn_kernel(AttnParams P) {
       __syncthreads();
       if (g < 0) break;
       const int hl = g / P.n_qb;
-      init_item(int(P.head_order[hl]), P.n_qb - 1 - (g - hl * P.n_qb));
+      init_item(int(P.head_order[hl]), P.n_qb - 1 - (g - hl * P.n_qb), -1);
       load_q();
       reset_acc();
       start_tiles();
       body();
-      merge_store(b, h, q0, vfac);
+      merge_store(b, h, q0, vfac, nullptr);
     }
   } else {
-    int hh, bq;
-    if (P.n_hl) {
-      const int r = int(blockIdx.x) >> 3;
-      if (r >= P.xcd_count[xcd]) return;
-      const int g = P.xcd_start[xcd] + r;
-      const int hl = g / P.n_qb;
-      hh = int(P.head_order[hl]);
-      bq = P.n_qb - 1 - (g - hl * P.n_qb);
-    } else {
-      // plain order: every (batch, head) pair; the host lists no item of a
-      // skipped head in the other modes
-      const int BH = P.batch * P.heads;
-      hh = int(blockIdx.x) % BH;
-      if (P.hd[hh % P.heads].kind == KIND_SKIP) return;
-      bq = P.n_qb - 1 - int(blockIdx.x) / BH;
-    }
-    init_item(hh, bq);
+    Item it;
+    if (!find_item(P, it)) return;
+    init_item(it.hh, it.bq, it.split);
     load_q();
     reset_acc();
     start_tiles();
     body();
-    merge_store(b, h, q0, vfac);
+    merge_store(b, h, q0, vfac, it.split >= 0 ? part_of<D>(P, it.part_row) : nullptr);
   }
 }
 
@@ -1114,21 +1162,9 @@ void attn_split_kernel(AttnParams P) {
   const int lr = lane >> 4;
   const int lc = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int xcd = blockIdx.x & 7;
-  int hh, bq;
-  if (P.n_hl) {
-    const int r = int(blockIdx.x) >> 3;
-    if (r >= P.xcd_count[xcd]) return;
-    const int g = P.xcd_start[xcd] + r;
-    const int hl = g / P.n_qb;
-    hh = int(P.head_order[hl]);
-    bq = P.n_qb - 1 - (g - hl * P.n_qb);
-  } else {
-    const int BH = P.batch * P.heads;
-    hh = int(blockIdx.x) % BH;
-    if (P.hd[hh % P.heads].kind == KIND_SKIP) return;
-    bq = P.n_qb - 1 - int(blockIdx.x) / BH;
-  }
+  Item it;
+  if (!find_item(P, it)) return;
+  const int hh = it.hh, bq = it.bq;
   const int b = hh / P.heads;
   const int h = hh - b * P.heads;
   const int kvh = h / P.kv_group;
@@ -1141,11 +1177,13 @@ void attn_split_kernel(AttnParams P) {
   TileSeq seq;
   item_tiles(P, kind, (int64_t(b) * P.idx_slots + P.hd[h].slot) * P.n_qb + bq, a0, a0 + nrows - 1,
              n_init, n_local, seq);
+  if (it.split >= 0)
+    seq.narrow(seq.total * it.split / P.n_split, seq.total * (it.split + 1) / P.n_split);
   const int total = seq.total;
-  const int mpos = min(seq.mpos, total);
+  const int mpos = max(min(seq.mpos, total), 0);
   const int64_t bk = int64_t(b) * (P.heads / P.kv_group) + kvh;
   const float vfac = __builtin_amdgcn_ldexpf(1.0f, load_uniform(P.vexp + bk));
-  const bool k_in_place = P.k_in_place;
+  const bool k_in_place = load_uniform(P.k_flag) != 0;
   const __amdgpu_buffer_rsrc_t krs =
       k_in_place
           ? __builtin_amdgcn_make_buffer_rsrc(
@@ -1424,6 +1462,7 @@ void attn_split_kernel(AttnParams P) {
   lanes_to_blocks(reduce_rows(l_g[0], l_g[1], l_g[2], l_g[3], RowSum()), l_b);
   rowsum[w][lane] = float2{l_b[0], l_b[1]};
   __syncthreads();
+  float* const pdst = it.split >= 0 ? part_of<D>(P, it.part_row) : nullptr;
   const float2 r0 = rowsum[0][lane], r1 = rowsum[1][lane], r2 = rowsum[2][lane],
                r3 = rowsum[3][lane];
 #pragma unroll
@@ -1431,6 +1470,11 @@ void attn_split_kernel(AttnParams P) {
     const float lt = hf ? (r0.y + r1.y) + (r2.y + r3.y) : (r0.x + r1.x) + (r2.x + r3.x);
     const float inv = lt > 0.0f ? vfac / lt : 0.0f;
     const int row = q0 + 32 * hf + (lane & 31);
+    if (pdst && w == 0 && lane < 32) {  // lane row 0 holds group 2 hf, lane row 1 group 2 hf + 1
+      float2* const ml = reinterpret_cast<float2*>(pdst + kBlock * D + 64 * hf) + lc;
+      if (lr == 0) *ml = make_float2(m_g[2 * hf], lt);
+      else ml[16] = make_float2(m_g[2 * hf + 1], lt);
+    }
     if (row >= P.s_q) continue;
     const int64_t obase = b * P.o_sb + int64_t(h) * P.o_sh + int64_t(row) * P.o_ss;
 #pragma unroll
@@ -1439,7 +1483,10 @@ void attn_split_kernel(AttnParams P) {
       for (int v = 0; v < 4; ++v) {
         const int d = 32 * (w * NW + nw) + 8 * v + 4 * (lane >> 5);
         const f32x16& x = o[nw][hf];
-        if constexpr (OUT_F32) {
+        if (pdst) {
+          store_out4<float>(pdst + (row - q0) * D + d, x[4 * v] * inv, x[4 * v + 1] * inv,
+                            x[4 * v + 2] * inv, x[4 * v + 3] * inv);
+        } else if constexpr (OUT_F32) {
           store_out4<float>(reinterpret_cast<float*>(P.o) + obase + d, x[4 * v] * inv,
                             x[4 * v + 1] * inv, x[4 * v + 2] * inv, x[4 * v + 3] * inv);
         } else {
@@ -1479,21 +1526,9 @@ void attn_wide_kernel(AttnParams P) {
   const int lr = lane >> 4;
   const int lc = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int xcd = blockIdx.x & 7;
-  int hh, bq;
-  if (P.n_hl) {
-    const int r = int(blockIdx.x) >> 3;
-    if (r >= P.xcd_count[xcd]) return;
-    const int g = P.xcd_start[xcd] + r;
-    const int hl = g / P.n_qb;
-    hh = int(P.head_order[hl]);
-    bq = P.n_qb - 1 - (g - hl * P.n_qb);
-  } else {
-    const int BH = P.batch * P.heads;
-    hh = int(blockIdx.x) % BH;
-    if (P.hd[hh % P.heads].kind == KIND_SKIP) return;
-    bq = P.n_qb - 1 - int(blockIdx.x) / BH;
-  }
+  Item it;
+  if (!find_item(P, it)) return;
+  const int hh = it.hh, bq = it.bq;
   const int b = hh / P.heads;
   const int h = hh - b * P.heads;
   const int kvh = h / P.kv_group;
@@ -1675,6 +1710,82 @@ void attn_wide_kernel(AttnParams P) {
       }
     }
   }
+}
+
+// Merge of the key splits of an item: O = sum_s w_s O_s, w_s = l_s 2^(m_s - M)
+// over their sum.  Four workgroups per (split pair, query block), 16 rows
+// each, thread = 4 dims of a row at a time; 4 * n_split * D bytes read per
+// row, bound by latency.
+template <typename T, bool OUT_F32, int D>
+__global__ __launch_bounds__(256) void attn_combine_kernel(CombineParams P) {
+  constexpr int TPR = D / 4;  // threads per row
+  constexpr int ROWS = kBlock / 4;
+  __shared__ float wt[kMaxSplit][ROWS];
+  const int item = int(blockIdx.x) >> 2, r0 = (int(blockIdx.x) & 3) * ROWS;
+  const int sp = item / P.n_qb, bq = item - sp * P.n_qb;
+  const int64_t stride = int64_t(P.n_qb) * (kBlock * (D + 2));  // between splits
+  const float* part = P.part + (int64_t(sp) * P.n_split * P.n_qb + bq) * (kBlock * (D + 2));
+  const int tid = threadIdx.x;
+  if (tid < ROWS) {
+    float m[kMaxSplit], l[kMaxSplit], M = -__builtin_inff(), L = 0.0f;
+#pragma unroll
+    for (int s = 0; s < kMaxSplit; ++s) {
+      const float2 x = s < P.n_split
+                           ? *reinterpret_cast<const float2*>(part + s * stride + kBlock * D + 2 * (r0 + tid))
+                           : make_float2(-1e30f, 0.0f);
+      m[s] = x.x;
+      l[s] = x.y;
+      M = fmaxf(M, x.x);
+    }
+#pragma unroll
+    for (int s = 0; s < kMaxSplit; ++s) {
+      l[s] *= __builtin_amdgcn_exp2f(m[s] - M);
+      L += l[s];
+    }
+    const float inv = L > 0.0f ? 1.0f / L : L;  // NaN stays NaN, no visible key gives 0
+#pragma unroll
+    for (int s = 0; s < kMaxSplit; ++s) wt[s][tid] = l[s] * inv;
+  }
+  __syncthreads();
+  const int pair = P.pair[sp];
+  const int b = pair / P.heads, h = pair - b * P.heads;
+  const int rows = min(ROWS, P.s_q - bq * kBlock - r0);
+  for (int i = tid; i < rows * TPR; i += 256) {
+    const int ri = i / TPR, d = 4 * (i - ri * TPR);
+    const int r = r0 + ri;
+    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int s = 0; s < P.n_split; ++s) {
+      const float4 x = *reinterpret_cast<const float4*>(part + s * stride + r * D + d);
+      const float f = wt[s][ri];
+      acc.x = __builtin_fmaf(f, x.x, acc.x);
+      acc.y = __builtin_fmaf(f, x.y, acc.y);
+      acc.z = __builtin_fmaf(f, x.z, acc.z);
+      acc.w = __builtin_fmaf(f, x.w, acc.w);
+    }
+    const int64_t off = b * P.o_sb + int64_t(h) * P.o_sh + int64_t(bq * kBlock + r) * P.o_ss + d;
+    if constexpr (OUT_F32) {
+      store_out4<float>(reinterpret_cast<float*>(P.o) + off, acc.x, acc.y, acc.z, acc.w);
+    } else {
+      store_out4_16<T>(reinterpret_cast<uint16_t*>(P.o) + off, acc.x, acc.y, acc.z, acc.w);
+    }
+  }
+}
+
+template <typename T, bool OUT_F32>
+static hipError_t launch_combine_t(const CombineParams& p, int D, hipStream_t st) {
+  const dim3 grid(uint32_t(p.n_pairs * p.n_qb * 4));
+  if (D == 64) hipLaunchKernelGGL((attn_combine_kernel<T, OUT_F32, 64>), grid, dim3(256), 0, st, p);
+  else if (D == 96) hipLaunchKernelGGL((attn_combine_kernel<T, OUT_F32, 96>), grid, dim3(256), 0, st, p);
+  else if (D == 128) hipLaunchKernelGGL((attn_combine_kernel<T, OUT_F32, 128>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((attn_combine_kernel<T, OUT_F32, 256>), grid, dim3(256), 0, st, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_combine(const CombineParams& p, int dtype, int out_dtype, int D, hipStream_t st) {
+  const bool f32 = out_dtype == 3;
+  if (dtype == Bf16::id)
+    return f32 ? launch_combine_t<Bf16, true>(p, D, st) : launch_combine_t<Bf16, false>(p, D, st);
+  return f32 ? launch_combine_t<F16, true>(p, D, st) : launch_combine_t<F16, false>(p, D, st);
 }
 
 // Workgroups of a launch of one item each: the longest XCD range on every XCD.

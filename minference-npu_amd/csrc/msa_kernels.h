@@ -69,28 +69,46 @@ struct HeadArg {
   float scale_log2;  // softmax scale * log2(e)
 };
 
+constexpr int kMaxEntries = 256;  // item-list entries of an attention launch
+constexpr int kMaxSplit = 8;      // key splits of one item
+
+// Merge of the key splits (attn_combine_kernel).
+struct CombineParams {
+  const float* part;
+  void* o;
+  int64_t o_sb, o_sh, o_ss;
+  int heads, s_q, n_qb, n_split, n_pairs;
+  uint8_t pair[kMaxHeads];  // (batch, head) of each split pair
+};
+
 struct AttnParams {
   const void* q;
   const void* k;
-  const uint16_t* kt;  // staged K operands (stage_kernel; unused when k_in_place)
+  const uint16_t* kt;  // staged K operands (stage_kernel; unused where k_flag is 1)
   const uint16_t* vt;  // staged V operands (stage_kernel)
   void* o;
   int64_t q_sb, q_sh, q_ss;
   int64_t k_sb, k_sh, k_ss;
   int64_t o_sb, o_sh, o_ss;
   int batch, heads, kv_group, s_q, s_k, n_qb, n_kb, s_pad;
-  // 1: the QK operands are read from k's own rows (every operand load is 16
-  // rows x 64 contiguous bytes) instead of the staged kt (see k_in_place)
-  int k_in_place;
+  // device flag the staging left: 1: the QK operands are read from k's own
+  // rows (every operand load is 16 rows x 64 contiguous bytes), 0: from kt
+  const int32_t* k_flag;
   const int32_t* idx;
   const int32_t* cnt;
   int idx_slots, topk_max;
   // Work items of this launch.  n_hl > 0: the items are (head_order[hl],
   // query block) for hl < n_hl, listed head-major with query blocks
   // longest-first; XCD x (workgroup i with i % 8 == x) takes items
-  // xcd_start[x] + (i / 8) for i / 8 < xcd_count[x].  n_hl == 0: every
-  // (batch, head) pair of the layer in plain order.
+  // xcd_start[x] + (i / 8) for i / 8 < xcd_count[x].  An entry is a (batch,
+  // head) pair (bits 0-7) or one key split of it (bit 31 set, bits 8-15: its
+  // index among the split pairs, bits 16-23: the split): the split takes its
+  // share of n_split of every query block's tiles and leaves the partial
+  // output in `part`.  n_hl == 0: every (batch, head) pair of the layer in
+  // plain order.
   int n_hl;
+  int n_split;
+  float* part;  // [split pair][split][query block]: 64 x D floats, 64 (m, l)
   int xcd_start[8];
   int xcd_count[8];
   int* queue;      // 8 counters of the XCD ranges (zeroed before each launch)
@@ -107,7 +125,7 @@ struct AttnParams {
   const uint16_t* gvt;
   int vs_slots, vs_cap, nv_pad;
   const int32_t* vexp;  // [batch * kv_heads]: staged V = V * 2^-vexp (stage_kernel)
-  int32_t head_order[kMaxHeads];
+  int32_t head_order[kMaxEntries];
   HeadArg hd[kMaxHeads];
 };
 static_assert(sizeof(AttnParams) <= 4096, "attention kernel arguments exceed 4 KB");
@@ -177,6 +195,7 @@ struct StageParams {
   // slot's kv head.  The attention kernel multiplies its output by 2^e.
   float* tmax;
   int32_t* vexp;
+  int32_t* k_flag;  // plain mode: set to 1 when K is left in its rows, else 0
   int16_t slot_kvh[kMaxHeads];
   // Fused pooling (plain mode): the first n_pool_wg workgroups of the launch
   // run the block estimator's pooling pass with these parameters.
@@ -261,6 +280,7 @@ hipError_t launch_vscale(const StageParams& p, int dtype, int D, hipStream_t st)
 hipError_t launch_decode(const DecodeParams& p, int dtype, int out_dtype, int D, hipStream_t st);
 hipError_t launch_attention(const AttnParams& p, int dtype, int out_dtype, int D,
                             hipStream_t st);
+hipError_t launch_combine(const CombineParams& p, int dtype, int out_dtype, int D, hipStream_t st);
 hipError_t launch_attention_vs(const AttnParams& p, int dtype, int out_dtype, int D,
                                hipStream_t st);
 hipError_t launch_vs_build(const VsBuildParams& p, int n_bs, hipStream_t st);

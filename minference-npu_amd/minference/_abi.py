@@ -53,7 +53,7 @@ MSA_ESTIMATE_SELECT_ONLY = 8
 
 MSA_MAX_HEADS = 128
 MSA_BLOCK = 64
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 _DTYPE_CODE = {
     torch.bfloat16: MSA_DTYPE_BF16,
@@ -83,6 +83,8 @@ EXPORTED_SYMBOLS = (
     "msa_rope_qk",
     "msa_round_f32",
     "msa_block_lists",
+    "msa_split_workspace_bytes",
+    "msa_layer_attention_split",
 )
 
 
@@ -253,6 +255,20 @@ def load_library() -> ctypes.CDLL:
         lib.msa_block_lists.argtypes = [
             ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64, ctypes.c_int64, ctypes.c_int32,
             ctypes.c_int32, ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p,
+            ctypes.c_void_p,
+        ]
+        lib.msa_split_workspace_bytes.restype = ctypes.c_size_t
+        lib.msa_split_workspace_bytes.argtypes = [
+            ctypes.POINTER(MsaTensor4), ctypes.POINTER(MsaTensor4), ctypes.POINTER(MsaHeadDesc),
+            ctypes.c_int32, ctypes.c_int32,
+        ]
+        lib.msa_layer_attention_split.restype = ctypes.c_int
+        lib.msa_layer_attention_split.argtypes = [
+            ctypes.POINTER(MsaTensor4), ctypes.POINTER(MsaTensor4),
+            ctypes.POINTER(MsaTensor4), ctypes.POINTER(MsaTensor4),
+            ctypes.POINTER(MsaHeadDesc), ctypes.c_int32,
+            ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32,
+            ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int32,
             ctypes.c_void_p,
         ]
         ver = lib.msa_abi_version()
@@ -532,7 +548,8 @@ def layer_attention(
     vs: Optional[tuple] = None,
     vs_ws: Optional[torch.Tensor] = None,
 ) -> None:
-    """Launch msa_layer_attention (or, with ``staged=True``,
+    """Launch msa_layer_attention (or msa_layer_attention_split where long items
+    are worth splitting over their keys; or, with ``staged=True``,
     msa_layer_attention_staged reading what msa_stage_kv staged in ``ws``
     for the same k and v).
     ``heads`` = [(kind, p1, p2, slot, scale)] * H.  With vertical_and_slash
@@ -572,6 +589,16 @@ def layer_attention(
             vs_ws.data_ptr(), vs_ws.numel(), ws.data_ptr(), ws.numel(), 0 if staged else 1,
             stream)
         check(st)
+        return
+    # few query blocks against a long key axis: room for key splits
+    split = lib.msa_split_workspace_bytes(ctypes.byref(qd), ctypes.byref(kd), arr, n,
+                                          int(topk_max))
+    if split:
+        split_ws = workspace(split, q.device)
+        check(lib.msa_layer_attention_split(
+            ctypes.byref(qd), ctypes.byref(kd), ctypes.byref(vd), ctypes.byref(od), arr, n,
+            idx_p, cnt_p, int(idx_slots), int(topk_max), split_ws.data_ptr(), split_ws.numel(),
+            ws.data_ptr(), ws.numel(), 0 if staged else 1, stream))
         return
     fn = lib.msa_layer_attention_staged if staged else lib.msa_layer_attention
     st = fn(
