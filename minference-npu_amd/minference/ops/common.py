@@ -48,9 +48,13 @@ def accepts_float32(names: Sequence[str], has_out: bool = True):
 
     def wrap(fn):
         sig = inspect.signature(fn)
+        first, at = names[0], list(sig.parameters).index(names[0])
 
         @functools.wraps(fn)
         def inner(*args, **kwargs):
+            t = args[at] if len(args) > at else kwargs.get(first)
+            if isinstance(t, torch.Tensor) and t.dtype != torch.float32:
+                return fn(*args, **kwargs)  # the usual call needs no binding of its arguments
             ba = sig.bind(*args, **kwargs)
             ts = [ba.arguments.get(n) for n in names]
             if not all(isinstance(t, torch.Tensor) and t.dtype == torch.float32 for t in ts):
@@ -187,7 +191,7 @@ def check_supported(q: torch.Tensor, k: torch.Tensor, v: Optional[torch.Tensor] 
             raise NotImplementedError(
                 f"the MI355X kernels take bf16 or fp16 inputs, got {t.dtype}"
             )
-    if len({t.dtype for t in tensors}) != 1:
+    if any(t.dtype != q.dtype for t in tensors):
         raise ValueError("q, k and v must share one dtype")
     if q.shape[-1] < 1:
         raise ValueError("head_dim must be positive")
@@ -200,9 +204,9 @@ def check_supported(q: torch.Tensor, k: torch.Tensor, v: Optional[torch.Tensor] 
 
 def kernel_view(t: torch.Tensor) -> torch.Tensor:
     """A view the kernels can read in place (D contiguous, 16-byte rows)."""
-    if t.stride(-1) != 1 or (t.data_ptr() % 16) != 0 or any(
-        (t.stride(i) * t.element_size()) % 16 for i in range(3) if t.shape[i] > 1
-    ):
+    es, st, sh = t.element_size(), t.stride(), t.shape
+    if (st[3] != 1 or t.data_ptr() % 16 or (st[0] * es % 16 and sh[0] > 1)
+            or (st[1] * es % 16 and sh[1] > 1) or (st[2] * es % 16 and sh[2] > 1)):
         return t.contiguous()
     return t
 
