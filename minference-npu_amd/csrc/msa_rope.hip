@@ -40,7 +40,7 @@ __device__ inline float val(uint16_t b) {
 // in flight.  A load or store instruction therefore covers up to 1 KB of
 // contiguous memory for the views of a fused qkv projection; the rotation
 // partner of a chunk (x[i +- rot/2]) comes from the lane rot/16 away.
-constexpr int kRopeTok = 16;
+constexpr int kRopeTok = 16;  // most tokens of a block
 constexpr int kRopeUnroll = 4;
 
 template <typename T>
@@ -105,12 +105,13 @@ __device__ inline u32x4 from_lane(const u32x4& v, int src_lane) {
   return r;
 }
 
-template <typename T>
+template <typename T, int TOK>
 __global__ __launch_bounds__(1024) void rope_kernel(const RopeParams P) {
-  __shared__ __attribute__((aligned(16))) uint16_t tab[kRopeTok * 2 * kRopeMaxRot];
+  static_assert(TOK <= kRopeTok, "tokens of a block");
+  __shared__ __attribute__((aligned(16))) uint16_t tab[TOK * 2 * kRopeMaxRot];
   const int64_t n_all = int64_t(P.batch) * P.s;
-  const int64_t tok0 = int64_t(blockIdx.x) * kRopeTok;
-  const int n_tok = int(min(int64_t(kRopeTok), n_all - tok0));
+  const int64_t tok0 = int64_t(blockIdx.x) * TOK;
+  const int n_tok = int(min(int64_t(TOK), n_all - tok0));
   const int b0 = int(tok0 / P.s);
   const int s0 = int(tok0 - int64_t(b0) * P.s);
   const int rc = P.rot / 8;  // 16-byte chunks per table row
@@ -183,17 +184,31 @@ __global__ __launch_bounds__(1024) void rope_kernel(const RopeParams P) {
 
 }  // namespace
 
-hipError_t launch_rope(const RopeParams& p, int dtype, hipStream_t st) {
+template <int TOK>
+static hipError_t launch_rope_t(const RopeParams& p, int dtype, hipStream_t st) {
   const int64_t n_tok = int64_t(p.batch) * p.s;
-  const dim3 grid(uint32_t((n_tok + kRopeTok - 1) / kRopeTok));
+  const dim3 grid(uint32_t((n_tok + TOK - 1) / TOK));
   const int hpw = 64 / (2 * p.n_pair + p.n_pass);
   const int n_groups = (p.heads + p.kv_heads + hpw - 1) / hpw;
   const dim3 block(uint32_t(64 * std::min(16, n_groups)));
   if (dtype == Bf16::id)
-    hipLaunchKernelGGL(rope_kernel<Bf16>, grid, block, 0, st, p);
+    hipLaunchKernelGGL((rope_kernel<Bf16, TOK>), grid, block, 0, st, p);
   else
-    hipLaunchKernelGGL(rope_kernel<F16>, grid, block, 0, st, p);
+    hipLaunchKernelGGL((rope_kernel<F16, TOK>), grid, block, 0, st, p);
   return hipGetLastError();
+}
+
+// Tokens of a block.  A block walks its tokens four at a time, so with few
+// tokens a block of 16 is a chain of four round trips on a part of the CUs;
+// with many, fewer tokens per block only read the tables more often.  Launch
+// times, 32 + 32 heads x 96, 16 / 4 / 1 tokens: 512 tokens 17.6 / 7.8 / 7.5 us,
+// 1000 18.4 / 8.8 / 11.9, 2000 19.5 / 14.7 / 21.7, 4000 22.2 / 24.9 / 37.9,
+// 32768 163 / 184 / 362.
+hipError_t launch_rope(const RopeParams& p, int dtype, hipStream_t st) {
+  const int64_t n_tok = int64_t(p.batch) * p.s;
+  if (n_tok >= 3072) return launch_rope_t<16>(p, dtype, st);
+  if (n_tok >= 512) return launch_rope_t<4>(p, dtype, st);
+  return launch_rope_t<1>(p, dtype, st);
 }
 
 }  // namespace msa
