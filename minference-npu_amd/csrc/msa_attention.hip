@@ -25,9 +25,10 @@
 //   v_mfma_f32_32x32x16_f16.  V is staged once per layer in exact operand
 //   order as fp16, so every V operand is one contiguous 1 KB load; K is read
 //   in place from the caller's rows (16 rows x 64 contiguous bytes per
-//   operand load) unless its rows overlap or a head's rows span more than a
-//   31-bit offset, or the launch is a vertical_and_slash one: then it is
-//   staged in operand order too.
+//   operand load) or staged in operand order too: where its rows overlap or
+//   a head's rows span more than a 31-bit offset, in vertical_and_slash
+//   launches, and where the row stride makes the in-place loads slow and the
+//   launch uses each key often enough (stage_k_mode).
 //   The exponentials are taken with each row's running max straight off
 //   QK, biased so that a row's maximum has P = 2^7 (P, O and the row sums
 //   all carry that factor, which cancels; it keeps small P out of fp16's
@@ -510,6 +511,53 @@ __device__ inline bool find_item(const AttnParams& P, Item& it) {
   return true;
 }
 
+// Workgroup barrier that orders LDS accesses only: __syncthreads would also
+// wait for the operand loads in flight.
+__device__ inline void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// The 64 query rows of an item as the QK B operand of every wave, through
+// LDS: wave w loads rows 16w .. 16w+15 as whole rows (1 KB per load, D / 32
+// loads), and each wave then reads the operands it needs.  Loaded straight
+// in operand order (16 rows x 64 bytes, all 64 rows by each wave) the same
+// rows cost 4 D / 32 loads per wave at 38 or 75 B/ns per CU, 1 to 2 us of the
+// L1 per item.  Before -> after: block ids at 32K of D = 64, short items, 255
+// -> 241 us; stream 16K of D = 256 604 -> 586; causal 8000 of D = 128 304 ->
+// 301; the 64K layer of D = 96, long items, 4508 -> 4479.
+template <int D>
+struct QTile {
+  static constexpr int NKS = D / 32;
+  static constexpr int LP = D + 8;  // padded LDS row (halves): operand reads free of conflicts
+  static constexpr int BYTES = kBlock * LP * 2;
+  // piece i of a lane: 16 bytes at row 16 w + r, element 8 c
+  __device__ static void load(const __amdgpu_buffer_rsrc_t& rs, int64_t row_stride, int w, int lane,
+                              u32x4 (&x)[NKS]) {
+#pragma unroll
+    for (int i = 0; i < NKS; ++i) {
+      const int f = lane + 64 * i, r = f / (D / 8), c = f - r * (D / 8);
+      x[i] = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     rs, uint32_t((16 * w + r) * row_stride * 2 + 16 * c), 0, 0));
+    }
+  }
+  __device__ static void put(uint16_t* tile, int w, int lane, const u32x4 (&x)[NKS]) {
+#pragma unroll
+    for (int i = 0; i < NKS; ++i) {
+      const int f = lane + 64 * i, r = f / (D / 8), c = f - r * (D / 8);
+      store16(tile + (16 * w + r) * LP + 8 * c, x[i]);
+    }
+  }
+  // lane (lc, lr) of group g, k-step ks: Q[16g + lc][32ks + 8lr .. +7]
+  __device__ static void operands(const uint16_t* tile, int lane, u32x4 (&qb)[4][NKS]) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks)
+        qb[g][ks] = load16(tile + (16 * g + (lane & 15)) * LP + 32 * ks + 8 * (lane >> 4));
+  }
+};
+
 // Partial output of a key split: 64 x D floats (each row normalised by its
 // own sum), then (m, l) of the 64 rows.
 template <int D>
@@ -680,12 +728,15 @@ void attn_kernel(AttnParams P) {
   };
 
   // ---- Q as the B operand: lane (lc, lr) of group g, k-step ks holds
-  // Q[q0 + 16g + lc][32ks + 8lr .. +7]; rows past S_q are zero
-  u32x4 qb[4][NKS];
+  // Q[q0 + 16g + lc][32ks + 8lr .. +7]; rows past S_q are zero or rows of the
+  // view (they feed only their own, never stored, outputs)
+  u32x4 qb[4][NKS], qx[NKS];
+  uint16_t* const qtile = reinterpret_cast<uint16_t*>(lds);  // until the merge
   auto load_q = [&]() INLINE {
     if constexpr (VS) {
       // vertical_and_slash: plain loads of row min(row, S_q - 1), rows past
-      // S_q zeroed after the load (fewer registers in this variant)
+      // S_q zeroed after the load (this variant has no registers left for
+      // rows in flight beside its lists: at D = 96 they spill)
       const uint16_t* qbase =
           reinterpret_cast<const uint16_t*>(P.q) + b * P.q_sb + int64_t(h) * P.q_sh;
 #pragma unroll
@@ -700,16 +751,14 @@ void attn_kernel(AttnParams P) {
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks)
           qb[g][ks] = q0 + 16 * g + lc < P.s_q ? qb[g][ks] : zero_u32x4();
-      return;
+    } else {
+      QTile<D>::load(qrs, P.q_ss, w, lane, qx);
     }
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const uint32_t roff = uint32_t((16 * g + lc) * P.q_ss * 2 + 16 * lr);
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks)
-        qb[g][ks] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(qrs, roff, 64 * ks, 0));
-    }
+  };
+  auto finish_q = [&]() INLINE {
+    QTile<D>::put(qtile, w, lane, qx);
+    lds_barrier();
+    QTile<D>::operands(qtile, lane, qb);
   };
 
   // K and V chunk operands of tile t: wave w reads chunk c = 4t + w.  Staged
@@ -996,6 +1045,7 @@ void attn_kernel(AttnParams P) {
     // part[((v * 3 + k) * 2 NDB + db * 2 + rb) * 64 + lane]: floats 4v .. 4v+3
     // of o[db][rb] of wave c (k = c < v ? c : c - 1) for owner v
     float4* part = reinterpret_cast<float4*>(lds + S::ML);
+    if constexpr (!VS) lds_barrier();  // every wave has read its Q operands
     ml[w * 64 + lane] = make_float4(m_b[0], m_b[1], l_b[0], l_b[1]);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -1104,6 +1154,7 @@ void attn_kernel(AttnParams P) {
     load_q();
     reset_acc();
     start_tiles();
+    finish_q();
     body();
     merge_store(b, h, q0, vfac, it.split >= 0 ? part_of<D>(P, it.part_row) : nullptr);
   }
@@ -1140,12 +1191,6 @@ struct SplitShape {
   static constexpr int NW = D / 128;  // output blocks of 32 dims per wave
 };
 
-// Workgroup barrier that orders LDS accesses only: __syncthreads would also
-// wait for the operand loads in flight.
-__device__ inline void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 template <typename T, bool OUT_F32, int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D > 128 ? 1 : 2)))
 void attn_split_kernel(AttnParams P) {
@@ -1156,6 +1201,7 @@ void attn_split_kernel(AttnParams P) {
   __shared__ float rowmax[4][64];                     // rare path: per wave, rows 0..63
   __shared__ float2 rowsum[4][64];                    // per wave and lane: sums of its two rows
   __shared__ int stamp[2];
+  __shared__ __align__(16) uint16_t qtile[QTile<D>::BYTES / 2];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1231,21 +1277,8 @@ void attn_split_kernel(AttnParams P) {
                        vrs, vo, ((4 * t + c) * NDB + w * NW + nw) * 1024, 0));
   };
 
-  u32x4 qb[4][NKS];
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const uint32_t roff = uint32_t((16 * g + lc) * P.q_ss * 2 + 16 * lr);
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks)
-      qb[g][ks] =
-          __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(qrs, roff, 64 * ks, 0));
-  }
-  if constexpr (D > 128) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) asm volatile("" : "+a"(qb[g][ks]));
-  }
+  u32x4 qb[4][NKS], qx[NKS];
+  QTile<D>::load(qrs, P.q_ss, w, lane, qx);
   f32x16 o[NW][2];
 #pragma unroll
   for (int nw = 0; nw < NW; ++nw)
@@ -1444,6 +1477,15 @@ void attn_split_kernel(AttnParams P) {
     load_k(t0, kr, false);
     load_v(t0, vr, false);
     pn = seq.fetch(3);
+    QTile<D>::put(qtile, w, lane, qx);
+    lds_barrier();
+    QTile<D>::operands(qtile, lane, qb);
+    if constexpr (D > 128) {  // Q in accumulation registers (the MFMA reads them there)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) asm volatile("" : "+a"(qb[g][ks]));
+    }
     qk(kr, sA, 0, NKS);
     load_k(t1, kr, total < 2);
     mask(sA, t0);
