@@ -86,8 +86,9 @@ __device__ inline int chunk_class(uint64_t m, int w, bool below_block) {
 }
 
 __global__ __launch_bounds__(256) void vs_build_kernel(VsBuildParams P) {
-  __shared__ uint32_t um[2 * kVsMaxTiles];  // per key tile: slash keys, then vertical keys
-  __shared__ uint32_t gm[2 * kVsMaxTiles];  // per gathered tile: gathered columns
+  extern __shared__ uint32_t masks[];
+  uint32_t* const um = masks;             // per key tile: slash keys, then vertical keys
+  uint32_t* const gm = um + 2 * P.n_kb;   // per gathered tile: gathered columns
   __shared__ int scratch[32];
   const int bq = blockIdx.x;
   const int bs = blockIdx.y;  // b * slots + slot
@@ -185,7 +186,9 @@ __global__ __launch_bounds__(256) void vs_build_kernel(VsBuildParams P) {
 }
 
 hipError_t launch_vs_build(const VsBuildParams& p, int n_bs, hipStream_t st) {
-  hipLaunchKernelGGL(vs_build_kernel, dim3(p.n_qb, n_bs), dim3(256), 0, st, p);
+  const int n_g = min((p.v_stride + kBlock - 1) / kBlock, kVsMaxTiles);
+  hipLaunchKernelGGL(vs_build_kernel, dim3(p.n_qb, n_bs), dim3(256),
+                     size_t(p.n_kb + n_g) * 8, st, p);
   return hipGetLastError();
 }
 
@@ -226,6 +229,30 @@ __device__ inline f32x4 mfma16<F16>(u32x2 a, u32x2 b, f32x4 c) {
                                                __builtin_bit_cast(f16x4, b), c, 0, 0, 0);
 }
 
+// Two floats rounded to T (nearest even), packed: one hardware conversion.
+typedef float f32x2p __attribute__((ext_vector_type(2)));
+template <typename T>
+__device__ inline uint32_t round2(float a, float b);
+template <>
+__device__ inline uint32_t round2<Bf16>(float a, float b) {
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2p{a, b}, b2));
+}
+template <>
+__device__ inline uint32_t round2<F16>(float a, float b) {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2p{a, b}, h2));
+}
+
+// x / d correctly rounded, with r = 1 / d correctly rounded (Markstein's
+// correction of x * r); tiny and non-finite x take the division itself.
+__device__ inline float div_by(float x, float d, float r) {
+  const float y = x * r;
+  const float z = __builtin_fmaf(__builtin_fmaf(-y, d, x), r, y);
+  const float ax = fabsf(x);
+  return ax > 0x1p-60f && ax < 0x1p100f ? z : x / d;
+}
+
 // Scores of the n last rows against 64 key columns.  Wave w takes rows
 // 16w .. 16w+15; per 16-key block, S^T = K . Q^T on the MFMA (lane l: keys
 // 4 (l / 16) + i, row l % 16) as 2 D / 32 partial sums of 16 exact products
@@ -239,13 +266,18 @@ __device__ inline f32x4 mfma16<F16>(u32x2 a, u32x2 b, f32x4 c) {
 // monotonic: when both ends of that interval round to the same value, it is
 // the rounding of the exact dot product (rounded to fp32 first); otherwise
 // (about 1 in 40 entries on N(0,1) data) the wave recomputes the dot
-// product exactly in fp64, 16 lanes per entry.
+// product exactly in fp64.  Its 16 rows x 64 keys are gathered in LDS first:
+// the ambiguous ones (about 26) then form one list, taken 16 at a time with 4
+// lanes and whole 16-byte loads each, and the results leave as 16-byte
+// stores.  What bounds it is the latency of those dependent steps: a list per
+// 16 keys, 16 lanes per entry and 4 entries at a time, took 356 us at 32K
+// tokens x 31 heads of D = 96, the hardware's packed rounding and a
+// multiplied reciprocal 331, this 258.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void vs_score_kernel(VsEstParams P) {
   constexpr int NKS = D / 32;
-  constexpr int DPL = D / 16;  // dims per lane of an exact dot product
-  __shared__ int32_t flist[4][256];  // per wave: flagged (row, key) of a key block
-  __shared__ uint16_t fres[4][256];
+  __shared__ uint16_t flist[4][1024];  // per wave: flagged (row << 6) | key
+  __shared__ __align__(16) uint16_t tile[4][16][kBlock + 8];  // per wave: rounded dot products
   const int j0 = blockIdx.x * kBlock;
   const int bs = blockIdx.y;
   const int b = bs / P.n_slots;
@@ -269,13 +301,14 @@ __global__ __launch_bounds__(256) void vs_score_kernel(VsEstParams P) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) qm[ks][e] = qa[ks][e] & kAbs;
   }
+  const float rinv = 1.0f / P.sqrt_d;
   const float c1 = 24.0f * 0x1p-23f * 1.01f;
   const float c0 = float(D + 2) * 0x1p-126f;
   uint16_t* xrow = P.x + int64_t(bs) * kBlock * P.s_pad;
-#pragma unroll 1
+  int nflag = 0;
+#pragma unroll
   for (int c = 0; c < 4; ++c) {
     const int key0 = j0 + 16 * c;
-    if (key0 >= P.s) break;
     const int ka = min(key0 + lc, P.s - 1);  // A operand: key row of this lane
     const uint16_t* krow = kb + int64_t(ka) * P.k_ss;
     const f32x4 zero = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -292,8 +325,7 @@ __global__ __launch_bounds__(256) void vs_score_kernel(VsEstParams P) {
       aacc = mfma_qk<T>(km, qm[ks], aacc);
     }
     // entries (key0 + 4 lr + i, row r); only existing ones are redone
-    uint16_t a16[4];
-    uint32_t redo = 0u;
+    uint32_t ends[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       float v = part[0][i];
@@ -301,68 +333,75 @@ __global__ __launch_bounds__(256) void vs_score_kernel(VsEstParams P) {
       for (int p = 1; p < 2 * NKS; ++p) v += part[p][i];
       // the +-bnd adds round too: 2 more 2^-23 units of sum |q_d k_d| >= |v|
       const float bnd = __builtin_fmaf(aacc[i], c1 + 2.0f * 0x1p-23f, c0);
-      const uint16_t lo = T::from_float(v - bnd), hi = T::from_float(v + bnd);
-      a16[i] = T::from_float(v);
-      if (lo != hi && r < n && key0 + 4 * lr + i < P.s) redo |= 1u << i;
+      ends[i] = round2<T>(v - bnd, v + bnd);
     }
-    // ambiguous entries: a wave-wide list, 16 lanes per exact dot product
-    int pos[4], nflag = 0;
+    // the lower end is the rounding of v too, unless the entry is redone
+    *reinterpret_cast<u32x2*>(&tile[w][lc][16 * c + 4 * lr]) =
+        u32x2{(ends[0] & 0xffffu) | (ends[1] << 16), (ends[2] & 0xffffu) | (ends[3] << 16)};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const bool f = (redo >> i) & 1u;
+      const bool f = (ends[i] & 0xffffu) != ends[i] >> 16 && r < n && key0 + 4 * lr + i < P.s;
       const uint64_t bal = __ballot(f);
-      pos[i] = nflag + __popcll(bal & ((1ull << lane) - 1ull));
-      if (f) flist[w][pos[i]] = (r << 17) | (key0 + 4 * lr + i);
+      if (f)
+        flist[w][nflag + __popcll(bal & ((1ull << lane) - 1ull))] =
+            uint16_t((lc << 6) | (16 * c + 4 * lr + i));
       nflag += __popcll(bal);
     }
-    if (nflag) {
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      const int grp = lane >> 4, sl = lane & 15;
-      for (int e0 = 0; e0 < nflag; e0 += 4) {
-        const int e = e0 + grp;
-        double dot = 0.0;
-        if (e < nflag) {
-          const int code = flist[w][e];
-          const uint16_t* qe = qb + int64_t(P.s - n + (code >> 17)) * P.q_ss + DPL * sl;
-          const uint16_t* ke = kb + int64_t(code & 0x1ffff) * P.k_ss + DPL * sl;
+  }
+  // ambiguous entries of the wave's 16 rows x 64 keys: 4 lanes per exact dot
+  // product, 16 of them at once
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  for (int e0 = 0; e0 < nflag; e0 += 16) {
+    const int e = e0 + (lane >> 2), sl = lane & 3;
+    const int code = flist[w][min(e, nflag - 1)];
+    const uint16_t* qe = qb + int64_t(P.s - n + 16 * w + (code >> 6)) * P.q_ss + 8 * sl;
+    const uint16_t* ke = kb + int64_t(j0 + (code & 63)) * P.k_ss + 8 * sl;
+    u32x4 qv[NKS], kv[NKS];
 #pragma unroll
-          for (int d = 0; d < DPL; d += 2) {
-            const uint32_t qw = *reinterpret_cast<const uint32_t*>(qe + d);
-            const uint32_t kw = *reinterpret_cast<const uint32_t*>(ke + d);
-            dot = __builtin_fma(double(T::to_float(uint16_t(qw & 0xffffu))),
-                                double(T::to_float(uint16_t(kw & 0xffffu))), dot);
-            dot = __builtin_fma(double(T::to_float(uint16_t(qw >> 16))),
-                                double(T::to_float(uint16_t(kw >> 16))), dot);
-          }
-        }
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
-        if (sl == 0 && e < nflag) fres[w][e] = T::from_float(float(dot));
-      }
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if ((redo >> i) & 1u) a16[i] = fres[w][pos[i]];
-      __builtin_amdgcn_wave_barrier();  // list reused by the next key block
+    for (int ks = 0; ks < NKS; ++ks) {
+      qv[ks] = load16(qe + 32 * ks);
+      kv[ks] = load16(ke + 32 * ks);
     }
-    if (r < n) {
-      uint16_t out[4];
+    double dot = 0.0;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int j = key0 + 4 * lr + i;
-        out[i] = j - (P.s - n) > r ? T::from_float(-__builtin_inff())
-                                   : T::from_float(T::to_float(a16[i]) / P.sqrt_d);
+    for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        dot = __builtin_fma(double(T::to_float(uint16_t(qv[ks][d] & 0xffffu))),
+                            double(T::to_float(uint16_t(kv[ks][d] & 0xffffu))), dot);
+        dot = __builtin_fma(double(T::to_float(uint16_t(qv[ks][d] >> 16))),
+                            double(T::to_float(uint16_t(kv[ks][d] >> 16))), dot);
       }
-      uint16_t* dst = xrow + int64_t(r) * P.s_pad + key0 + 4 * lr;
-      if (key0 + 4 * lr + 3 < P.s) {  // 4 keys, 8-byte aligned (s_pad and key0 + 4 lr are)
-        *reinterpret_cast<uint2*>(dst) = uint2{uint32_t(out[0]) | (uint32_t(out[1]) << 16),
-                                               uint32_t(out[2]) | (uint32_t(out[3]) << 16)};
+    dot += __shfl_xor(dot, 1, 64);
+    dot += __shfl_xor(dot, 2, 64);
+    if (sl == 0 && e < nflag) tile[w][code >> 6][code & 63] = T::from_float(float(dot));
+  }
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  // x = dot / sqrt(D), masked: 8 lanes per row, 8 keys each
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const int row = 8 * m + (lane >> 3), ro = 16 * w + row, k0 = j0 + 8 * (lane & 7);
+    const u32x4 dv = *reinterpret_cast<const u32x4*>(&tile[w][row][8 * (lane & 7)]);
+    float x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      x[i] = k0 + i - (P.s - n) > ro
+                 ? -__builtin_inff()
+                 : div_by(T::to_float(uint16_t(i & 1 ? dv[i / 2] >> 16 : dv[i / 2] & 0xffffu)),
+                          P.sqrt_d, rinv);
+    u32x4 out;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out[i] = round2<T>(x[2 * i], x[2 * i + 1]);
+    if (ro < n) {
+      uint16_t* dst = xrow + int64_t(ro) * P.s_pad + k0;
+      if (k0 + 7 < P.s) {  // 16-byte aligned (s_pad and j0 are multiples of 64)
+        store16(dst, out);
       } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (key0 + 4 * lr + i < P.s) dst[i] = out[i];
+        for (int i = 0; i < 8; ++i)
+          if (k0 + i < P.s) dst[i] = uint16_t(i & 1 ? out[i / 2] >> 16 : out[i / 2] & 0xffffu);
       }
     }
   }
@@ -501,38 +540,20 @@ __global__ __launch_bounds__(256) void vs_sums_kernel(VsEstParams P) {
   P.slash[int64_t(bs) * P.s + t] = fs;
 }
 
-// Block-wide exclusive prefix of a 0/1 flag over NT threads (see
-// block_prefix).
-template <int NT>
-__device__ inline int block_prefix_n(bool flag, int* scratch, int* total) {
-  constexpr int NW = NT / 64;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const uint64_t bal = __ballot(flag);
-  const int in_wave = __popcll(bal & ((1ull << lane) - 1ull));
-  if (lane == 0) scratch[w] = __popcll(bal);
-  __syncthreads();
-  int before = 0, all = 0;
-#pragma unroll
-  for (int v = 0; v < NW; ++v) {
-    before += v < w ? scratch[v] : 0;
-    all += scratch[v];
-  }
-  __syncthreads();
-  *total = all;
-  return before + in_wave;
-}
-
 // Top-k of one score row (y = 0: vertical, y = 1: slash): the k-th largest
 // key T by a 32-step bitwise search (the largest T with at least k keys >= T;
 // non-negative floats order like their bits), counting with wave ballots
 // (no atomics: the keys share their leading bits), then every key above T and
 // the lowest-index keys equal to T, in index order.  The first 64K keys stay
-// in registers across the passes.
+// in registers across the search.  The output takes one scan of all the
+// (64-key run) counts; a scan per 1024 keys took 86 us at 32K keys, this 68.
 constexpr int kTopkThreads = 1024;
 constexpr int kTopkRegs = 64;  // keys per thread held in registers
 
 __global__ __launch_bounds__(kTopkThreads) void vs_topk_kernel(VsEstParams P) {
   __shared__ int scratch[kTopkThreads / 64];
+  __shared__ int2 counts[kTopkThreads], wsum[kTopkThreads / 64];
+  static_assert(kTopkRegs * (kTopkThreads / 64) == kTopkThreads, "one count per thread");
   const int bs = blockIdx.x;
   const int slot = bs % P.n_slots;
   const bool is_slash = blockIdx.y == 1;
@@ -568,20 +589,57 @@ __global__ __launch_bounds__(kTopkThreads) void vs_topk_kernel(VsEstParams P) {
   }
   const int need_eq = kk0 - count_ge(t + 1u);  // keys equal to t to take
   int32_t* out = is_slash ? P.s_idx + int64_t(bs) * P.s_stride : P.v_idx + int64_t(bs) * P.v_stride;
-  int taken = 0, eq_seen = 0;
-  for (int i0 = 0; i0 < P.s; i0 += kTopkThreads) {
-    const int i = i0 + tid;
-    const uint32_t key = i < P.s ? keys[i] : 0u;
-    const bool gt = i < P.s && key > t;
-    const bool eq = i < P.s && key == t;
-    int n_eq;
-    const int eq_rank = eq_seen + block_prefix_n<kTopkThreads>(eq, scratch, &n_eq);
-    const bool take = gt || (eq && eq_rank < need_eq);
-    int n_take;
-    const int pos = taken + block_prefix_n<kTopkThreads>(take, scratch, &n_take);
-    if (take) out[pos] = is_slash ? P.s - 1 - i : i;
-    taken += n_take;
-    eq_seen += n_eq;
+  // Output in index order.  Keys i = 64 (16 m + w) + lane: one count per
+  // (m, w) of the keys above t and equal to it, one scan of all of them, and
+  // each wave places its keys from its counts' offsets.
+  int gt_base = 0, eq_base = 0;
+  for (int m0 = 0; kTopkThreads * m0 < P.s; m0 += kTopkRegs) {
+    // the keys are read again here (from the L2): 64 ballots kept in flight
+    // over the registers spill
+    const int n_m = min((P.s - kTopkThreads * m0 + kTopkThreads - 1) / kTopkThreads, kTopkRegs);
+    counts[tid] = make_int2(0, 0);
+    __syncthreads();
+#pragma unroll 4
+    for (int m = 0; m < n_m; ++m) {
+      const int i = tid + kTopkThreads * (m0 + m);
+      const uint32_t key = i < P.s ? keys[i] : 0u;
+      const uint64_t g = __ballot(i < P.s && key > t), q = __ballot(i < P.s && key == t);
+      if (lane == 0) counts[16 * m + w] = make_int2(__popcll(g), __popcll(q));
+    }
+    __syncthreads();
+    int2 c = counts[tid], in = c;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int g = __shfl_up(in.x, off, 64), q = __shfl_up(in.y, off, 64);
+      if (lane >= off) { in.x += g; in.y += q; }
+    }
+    if (lane == 63) wsum[w] = in;
+    __syncthreads();
+    int2 before = make_int2(gt_base, eq_base);
+#pragma unroll
+    for (int v = 0; v < kTopkThreads / 64; ++v) {
+      const int2 ws = wsum[v];
+      if (v < w) { before.x += ws.x; before.y += ws.y; }
+      gt_base += ws.x;
+      eq_base += ws.y;
+    }
+    counts[tid] = make_int2(before.x + in.x - c.x, before.y + in.y - c.y);
+    __syncthreads();
+#pragma unroll 4
+    for (int m = 0; m < n_m; ++m) {
+      const int i = tid + kTopkThreads * (m0 + m);
+      const uint32_t key = i < P.s ? keys[i] : 0u;
+      const bool gt = i < P.s && key > t, eq = i < P.s && key == t;
+      const uint64_t bg = __ballot(gt), bq = __ballot(eq);
+      if ((bg | bq) != 0ull) {
+        const int2 base = counts[16 * m + w];
+        const uint64_t below = (1ull << lane) - 1ull;
+        const int eq_rank = base.y + __popcll(bq & below);
+        const int pos = base.x + __popcll(bg & below) + min(eq_rank, need_eq);
+        if (gt || (eq && eq_rank < need_eq)) out[pos] = is_slash ? P.s - 1 - i : i;
+      }
+    }
+    __syncthreads();  // counts reused by the next 64K keys
   }
   if (tid == 0) (is_slash ? P.s_cnt : P.v_cnt)[bs] = kk0;
 }
