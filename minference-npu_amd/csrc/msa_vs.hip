@@ -34,11 +34,6 @@ namespace msa {
 
 constexpr int kVsMaxTiles = kVsMaxSeq / kBlock;
 
-__device__ inline uint64_t bit_range(int a, int b) {  // bits [a, b), 0 <= a < b <= 64
-  const uint64_t hi = b >= 64 ? ~0ull : ((1ull << b) - 1ull);
-  return hi & ~((1ull << a) - 1ull);
-}
-
 __device__ inline void lds_or64(uint32_t* m, int t, uint64_t v) {
   if (uint32_t(v)) atomicOr(&m[2 * t], uint32_t(v));
   if (uint32_t(v >> 32)) atomicOr(&m[2 * t + 1], uint32_t(v >> 32));
@@ -85,10 +80,15 @@ __device__ inline int chunk_class(uint64_t m, int w, bool below_block) {
   return c == 0u ? 0 : (c == 0xffffu && below_block ? 1 : 2);
 }
 
+// Bounded by its LDS atomics, barriers and the blocks in flight: at 32K tokens
+// x 31 heads 188 us with masks for the longest sequence in LDS (four blocks
+// per CU) and up to four atomics per window, 171 with LDS sized by the call,
+// 105 with one atomic per window and one barrier for the first pass.
 __global__ __launch_bounds__(256) void vs_build_kernel(VsBuildParams P) {
   extern __shared__ uint32_t masks[];
-  uint32_t* const um = masks;             // per key tile: slash keys, then vertical keys
-  uint32_t* const gm = um + 2 * P.n_kb;   // per gathered tile: gathered columns
+  uint32_t* const um = masks;                  // per key tile: slash keys, then vertical keys
+  uint32_t* const hm = um + 2 * P.n_kb;        // per key tile: last keys of slash windows
+  uint32_t* const gm = hm + 2 * P.n_kb + 2;    // per gathered tile: gathered columns
   __shared__ int scratch[32];
   const int bq = blockIdx.x;
   const int bs = blockIdx.y;  // b * slots + slot
@@ -101,22 +101,31 @@ __global__ __launch_bounds__(256) void vs_build_kernel(VsBuildParams P) {
   const int32_t* vrow = P.v_idx + int64_t(bs) * P.v_stride;
   const int32_t* srow = P.s_idx + int64_t(bs) * P.s_stride;
 
-  for (int i = tid; i < 2 * n_t; i += 256) um[i] = 0u;
+  for (int i = tid; i < 2 * n_t + 2; i += 256) hm[i] = 0u;
   for (int i = tid; i < 2 * n_g; i += 256) gm[i] = 0u;
   __syncthreads();
 
-  // slash windows, clipped to the keys the block's rows can reach
+  // slash windows: 64 keys ending at hi (or from key 0 on), of which the keys
+  // the block's rows can reach count.  Each window marks its last key; tile
+  // t's keys up to the last mark of its own and after the first mark of tile
+  // t + 1 are in some window.  One atomic per window, not one per 32 keys:
+  // neighbouring windows meet in the same words.
   const int kend = min(end_m, P.s_k);
   for (int i = tid; i < ns; i += 256) {
     const int64_t s = srow[i];
     if (s >= end_m) continue;
-    const int hi = int(min(max(int64_t(end_m) - s, int64_t(kBlock)), int64_t(P.s_k)));
-    const int lo = max(hi - kBlock, 0);
-    const int hc = min(hi, kend);
-    if (lo >= hc) continue;
-    const int t0 = lo / kBlock, t1 = (hc - 1) / kBlock;
-    for (int t = t0; t <= t1; ++t)
-      lds_or64(um, t, bit_range(max(lo, kBlock * t) - kBlock * t, min(hc, kBlock * t + kBlock) - kBlock * t));
+    const int last = int(min(max(int64_t(end_m) - s, int64_t(kBlock)), int64_t(P.s_k))) - 1;
+    if (last < kBlock * (n_t + 1)) atomicOr(&hm[last >> 5], 1u << (last & 31));
+  }
+  __syncthreads();
+  for (int t = tid; t < n_t; t += 256) {
+    const uint64_t own = lds_get64(hm, t), next = lds_get64(hm, t + 1);
+    uint64_t m = own ? ~0ull >> __builtin_clzll(own) : 0ull;
+    if (next) m |= ~((2ull << __builtin_ctzll(next)) - 1ull);
+    const int vis = kend - kBlock * t;  // keys of the tile before kend
+    if (vis < kBlock) m &= (1ull << vis) - 1ull;
+    um[2 * t] = uint32_t(m);
+    um[2 * t + 1] = uint32_t(m >> 32);
   }
   __syncthreads();
 
@@ -143,14 +152,16 @@ __global__ __launch_bounds__(256) void vs_build_kernel(VsBuildParams P) {
     const bool gat = e >= n_t;
     const uint64_t m = e < n_t ? lds_get64(um, e) : (e < n_t + n_g ? lds_get64(gm, e - n_t) : 0ull);
     const bool below = gat || e < bq;
-    bool f[4];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) f[w] = chunk_class(m, w, below) == 1;
-    int pre[4], tot[4];
-    block_prefix<4>(f, scratch, pre, tot);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) n_un[w] += tot[w];
+    for (int w = 0; w < 4; ++w) n_un[w] += __popcll(__ballot(chunk_class(m, w, below) == 1));
   }
+  if ((tid & 63) == 0)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) scratch[4 * (tid >> 6) + w] = n_un[w];
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 4; ++w) n_un[w] = scratch[w] + scratch[4 + w] + scratch[8 + w] + scratch[12 + w];
+  __syncthreads();
   // pass 2: the entries, unmasked from 0 and masked from n_un[w] in each
   // wave's list
   uint32_t* lists = P.lists + row * 4 * P.cap;
@@ -188,7 +199,7 @@ __global__ __launch_bounds__(256) void vs_build_kernel(VsBuildParams P) {
 hipError_t launch_vs_build(const VsBuildParams& p, int n_bs, hipStream_t st) {
   const int n_g = min((p.v_stride + kBlock - 1) / kBlock, kVsMaxTiles);
   hipLaunchKernelGGL(vs_build_kernel, dim3(p.n_qb, n_bs), dim3(256),
-                     size_t(p.n_kb + n_g) * 8, st, p);
+                     size_t(2 * p.n_kb + 1 + n_g) * 8, st, p);
   return hipGetLastError();
 }
 
