@@ -522,7 +522,7 @@ __device__ inline void lds_barrier() {
 // loads), and each wave then reads the operands it needs.  Loaded straight
 // in operand order (16 rows x 64 bytes, all 64 rows by each wave) the same
 // rows cost 4 D / 32 loads per wave at 38 or 75 B/ns per CU, 1 to 2 us of the
-// L1 per item.  Before -> after: block ids at 32K of D = 64, short items, 255
+// L1 per item.  Before -> after: block ids at 32K of D = 128, short items, 255
 // -> 241 us; stream 16K of D = 256 604 -> 586; causal 8000 of D = 128 304 ->
 // 301; the 64K layer of D = 96, long items, 4508 -> 4479.
 template <int D>

@@ -7,7 +7,7 @@
 //
 // Bound by HBM: K and V are read once, 4*D bytes per key and kv head.  Two
 // kernels, chosen by the heads that share a kv head: decode_kernel (one head,
-// VALU) and decode_group_kernel (two or more, matrix cores).  On one box:
+// VALU) and decode_group_kernel (two or more, matrix cores).  Measured:
 // 32 heads on 32 kv heads x 96, 65536 keys: 127.5 us VALU, 141 us matrix
 // cores (at D = 96 a quarter of its V lanes have no dims to read); 8 x 32
 // heads on 8 kv heads x 128, 16384 keys: 200.8 us VALU (every head reads its
