@@ -500,7 +500,8 @@ def stage_kv_pool(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                   slot_heads: Sequence[int], est_ws: Optional[torch.Tensor],
                   ws: torch.Tensor) -> None:
     """Launch msa_stage_kv_pool on the current stream: V (and K where the
-    attention kernel cannot read it in place) staged into ``ws`` and, for the block slots ``slot_heads``, Q and K pooled into ``est_ws``
+    attention kernel does not read it in place) staged into ``ws`` and, for
+    the block slots ``slot_heads``, Q and K pooled into ``est_ws``
     (the workspace of the MSA_ESTIMATE_SELECT_ONLY block_estimate call that
     follows)."""
     n = len(slot_heads)
