@@ -321,19 +321,28 @@ void decode_group_kernel(DecodeParams P) {
   const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<unsigned char*>(vbase), short(0), int(int64_t(P.s_k) * P.v_ss * 2), 0x00020000);
   const uint32_t kss = uint32_t(P.k_ss) * 2u, vss = uint32_t(P.v_ss) * 2u;  // row bytes
-  const uint32_t koff = uint32_t(lc) * kss + 16u * lr;
-  // D = 64, 96: lanes past the row's last dim read nothing
-  const uint32_t voff = 8 * lc < D ? uint32_t(4 * lr) * vss + 16u * lc : 0x80000000u;
+  // A block's key rows sit in the lane offsets and the scalar offset names its
+  // first key, j0 < S: the range check compares the lane offset with the
+  // records left behind the scalar offset, so that one must stay inside them.
+  // D = 64, 96: lanes past the row's last dim read nothing.
+  uint32_t koff[U], voff[U][4];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    koff[u] = uint32_t(16 * u + lc) * kss + 16u * lr;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      voff[u][i] = 8 * lc < D ? uint32_t(16 * u + 4 * lr + i) * vss + 16u * lc : 0x80000000u;
+  }
   // K and V are read once per call: loads carry the non-temporal hint (cache
   // policy bit 1) so the stream does not evict reused lines.
   auto load_block = [&](int j0, u32x4 (&kr)[U][NKS], u32x4 (&vr)[U][4][VG]) INLINE {
+    const int ks0 = j0 * int(kss), vs0 = j0 * int(vss);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int ks0 = (j0 + 16 * u) * int(kss);
 #pragma unroll
       for (int ks = 0; ks < NKS; ++ks)
         kr[u][ks] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(krs, koff, ks0 + 64 * ks, 2));
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(krs, koff[u], ks0 + 64 * ks, 2));
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -342,8 +351,7 @@ void decode_group_kernel(DecodeParams P) {
 #pragma unroll
         for (int g = 0; g < VG; ++g)
           vr[u][i][g] = __builtin_bit_cast(
-              u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                         vrs, voff, (j0 + 16 * u + i) * int(vss) + 256 * g, 2));
+              u32x4, __builtin_amdgcn_raw_buffer_load_b128(vrs, voff[u][i], vs0 + 256 * g, 2));
   };
 
   // o[g][e]: lane (lc, lr) holds head lc, dims 128 g + 8 (4 lr + j) + e

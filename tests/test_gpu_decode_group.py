@@ -57,3 +57,26 @@ def test_row_stride_and_late_maximum(gpu_device):
     _check(gpu_device, 1, 4, 1, 900, 96, torch.bfloat16, k_pad=40)
     _check(gpu_device, 1, 4, 2, 2000, 128, torch.bfloat16,
            boost=[(3, 3.0), (700, 8.0), (1500, 30.0), (1999, 60.0)])
+
+
+# Rows past the cache's end: the last 16- or 32-key block of a wave reaches
+# over S (by up to 31 rows), and those rows must read as zeros, whatever lies
+# there.  The rows past S are NaN here, where 0 * NaN would show.
+@pytest.mark.parametrize("H,Hkv", [(4, 1)])
+@pytest.mark.parametrize("S", [1, 3, 15, 16, 17, 33, 64, 129, 1041])
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (96, torch.float16),
+                                     (128, torch.bfloat16), (256, torch.float16),
+                                     (512, torch.bfloat16)])
+def test_rows_past_the_cache_read_as_zeros(gpu_device, H, Hkv, S, D, dtype):
+    from minference.backend.attention import decode_dense
+
+    g = torch.Generator(gpu_device).manual_seed(S + D)
+    q = torch.randn(2, H, 1, D, device=gpu_device, generator=g).to(dtype)
+    k, v = (torch.randn(2, Hkv, S + 64, D, device=gpu_device, generator=g).to(dtype)
+            for _ in range(2))
+    k[:, :, S:], v[:, :, S:] = float("nan"), float("nan")
+    ks, vs = k[:, :, :S], v[:, :, :S]
+    out = decode_dense(q, ks, vs, out=torch.empty(q.shape, device=gpu_device))
+    x = q.double() @ ks.double().repeat_interleave(H // Hkv, 1).transpose(-1, -2).contiguous()
+    ref = torch.softmax(x / D ** 0.5, -1) @ vs.double().repeat_interleave(H // Hkv, 1)
+    assert float((out - ref).abs().max()) < 1e-5  # the bound above
