@@ -169,11 +169,12 @@ __global__ __launch_bounds__(256) void decode_kernel(DecodeParams P) {
 
   // Wave w takes blocks first + 64 i, i < nblk, two blocks in flight ahead
   // of the one being reduced, in three rotating register sets.  Loads past
-  // the wave's last block repeat that block, so every load is unconditional
-  // and in range.
+  // the wave's last block repeat that block (a wave without any loads the
+  // chunk's first), so every load is unconditional and starts below S, as the
+  // range check of a scalar offset needs.
   const int first = j_begin + 16 * w;
   const int nblk = j_end > first ? (j_end - first + 63) / 64 : 0;
-  const int last = first + 64 * max(nblk - 1, 0);
+  const int last = nblk > 0 ? first + 64 * (nblk - 1) : j_begin;
   auto jb = [&](int i) { return min(first + 64 * i, last); };
   u32x4 ka[NL], va[NL], kb[NL], vb[NL], kc[NL], vc[NL];
   load_block(jb(0), ka, va);

@@ -61,8 +61,9 @@ def test_row_stride_and_late_maximum(gpu_device):
 
 # Rows past the cache's end: the last 16- or 32-key block of a wave reaches
 # over S (by up to 31 rows), and those rows must read as zeros, whatever lies
-# there.  The rows past S are NaN here, where 0 * NaN would show.
-@pytest.mark.parametrize("H,Hkv", [(4, 1)])
+# there.  The rows past S are NaN here, where 0 * NaN would show.  (2, 2): the
+# kernel for one head per kv head, whose waves can be left without a block.
+@pytest.mark.parametrize("H,Hkv", [(4, 1), (2, 2)])
 @pytest.mark.parametrize("S", [1, 3, 15, 16, 17, 33, 64, 129, 1041])
 @pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (96, torch.float16),
                                      (128, torch.bfloat16), (256, torch.float16),
