@@ -361,8 +361,10 @@ void decode_group_kernel(DecodeParams P) {
   for (int g = 0; g < VG; ++g)
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[g][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  float m = -1e30f;  // running max of head lc (scaled, log2 units), the same in its 4 lanes
-  float l = 0.0f;    // this lane's share of the sum
+  // running max of head lc (scaled, log2 units), the same in its 4 lanes, and
+  // what P is taken against: m, or 0 as long as the head has no score above -inf
+  float m = -__builtin_inff(), mp = 0.0f;
+  float l = 0.0f;  // this lane's share of the sum
   const float c = P.scale_log2;
 
   auto block = [&](int j0, const u32x4 (&kr)[U][NKS], const u32x4 (&vr)[U][4][VG]) INLINE {
@@ -383,7 +385,8 @@ void decode_group_kernel(DecodeParams P) {
     bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
     if (__ballot(bm > m + kSlack) != 0) {
       const float mn = fmaxf(m, bm);
-      const float al = __builtin_amdgcn_exp2f(m - mn);
+      mp = mn == -__builtin_inff() ? 0.0f : mn;
+      const float al = __builtin_amdgcn_exp2f(m - mp);  // m = -inf at first: 0
       m = mn;
       l *= al;
 #pragma unroll
@@ -395,7 +398,7 @@ void decode_group_kernel(DecodeParams P) {
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float p = __builtin_amdgcn_exp2f(s[u][i] - m);
+        const float p = __builtin_amdgcn_exp2f(s[u][i] - mp);
         l += p;
 #pragma unroll
         for (int g = 0; g < VG; ++g)
@@ -444,13 +447,13 @@ void decode_group_kernel(DecodeParams P) {
     // thread: 4 dims of head tid / 32, then of head 8 + tid / 32
     const int d = 128 * g + 4 * (tid & 31);
     for (int hd = tid >> 5; hd < nh && d < D; hd += 8) {
-      float M = -1e30f, L = 0.0f, f[4];
+      float M = -__builtin_inff(), L = 0.0f, f[4];
 #pragma unroll
       for (int v = 0; v < 4; ++v) M = fmaxf(M, sm[v][hd]);
       float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        f[v] = __builtin_amdgcn_exp2f(sm[v][hd] - M);
+        f[v] = M == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(sm[v][hd] - M);
         L += f[v] * sl[v][hd];
         const float4 x = *reinterpret_cast<const float4*>(&om[v][hd][4 * (tid & 31)]);
         acc.x = __builtin_fmaf(f[v], x.x, acc.x);

@@ -81,3 +81,53 @@ def test_rows_past_the_cache_read_as_zeros(gpu_device, H, Hkv, S, D, dtype):
     x = q.double() @ ks.double().repeat_interleave(H // Hkv, 1).transpose(-1, -2).contiguous()
     ref = torch.softmax(x / D ** 0.5, -1) @ vs.double().repeat_interleave(H // Hkv, 1)
     assert float((out - ref).abs().max()) < 1e-5  # the bound above
+
+
+# Scores far below zero, down to the lowest finite ones: a row's softmax is of
+# their differences, so the key with the smallest magnitude takes all of it.
+# (2, 2): one head per kv head.
+@pytest.mark.parametrize("H,Hkv", [(4, 1), (17, 1), (2, 2)])
+@pytest.mark.parametrize("S", [1, 16, 33, 700])
+@pytest.mark.parametrize("e", [55, 60, 62])  # scores about -2^(2e - 3), log2(1e30) is 99.7
+def test_low_scores(gpu_device, H, Hkv, S, e):
+    from minference.backend.attention import decode_dense
+
+    D = 64
+    g = torch.Generator(gpu_device).manual_seed(S)
+    q = torch.zeros(1, H, 1, D, device=gpu_device, dtype=torch.bfloat16)
+    k = torch.zeros(1, Hkv, S, D, device=gpu_device, dtype=torch.bfloat16)
+    v = torch.randn(1, Hkv, S, D, device=gpu_device, generator=g).to(torch.bfloat16)
+    q[..., 5] = 2.0 ** e
+    k[..., 5] = -(2.0 ** e)
+    top = (7 * S) // 11
+    k[:, :, top, 5] = -(2.0 ** (e - 1))
+    out = decode_dense(q, k, v, out=torch.empty(q.shape, device=gpu_device))
+    want = v[:, :, top].float().repeat_interleave(H // Hkv, 1)
+    assert torch.equal(out[:, :, 0], want)
+
+
+def test_infinite_scores(gpu_device):
+    """-inf scores weigh nothing, wherever they stand; a row of nothing else
+    gives 0, NaN stays with its own head."""
+    from minference.backend.attention import decode_dense
+
+    D, S = 64, 300
+    g = torch.Generator(gpu_device).manual_seed(3)
+    q = torch.randn(1, 4, 1, D, device=gpu_device, generator=g).to(torch.bfloat16)
+    q[..., 0] = torch.tensor([1.0, 1.0, 1.0, 2.0], device=gpu_device)[:, None]
+    k, v = (torch.randn(1, 1, S, D, device=gpu_device, generator=g).to(torch.bfloat16)
+            for _ in range(2))
+    low = torch.arange(S, device=gpu_device) % 40 != 17  # whole 16- and 32-key blocks among them
+    k[:, :, low, 0] = -float("inf")
+    out = decode_dense(q, k, v, out=torch.empty(q.shape, device=gpu_device))
+    x = q.double() @ k[:, :, ~low].double().transpose(-1, -2).contiguous() / D ** 0.5
+    ref = torch.softmax(x, -1) @ v[:, :, ~low].double()
+    assert float((out - ref).abs().max()) < 1e-5
+    k[..., 0] = -float("inf")
+    assert not decode_dense(q, k, v).any()
+    # V: an infinite value reaches its own dim of every head and no other
+    k = torch.randn(1, 1, S, D, device=gpu_device, generator=g).to(torch.bfloat16)
+    v[0, 0, 211, 9] = float("inf")
+    out = decode_dense(q, k, v)
+    assert torch.isinf(out[..., 9]).all()
+    assert torch.isfinite(out[..., :9]).all() and torch.isfinite(out[..., 10:]).all()
