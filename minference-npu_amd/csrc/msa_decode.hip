@@ -148,9 +148,10 @@ __global__ __launch_bounds__(256) void decode_kernel(DecodeParams P) {
     for (int off = 8; off > 0; off >>= 1) bm = fmaxf(bm, __shfl_xor(bm, off, 64));
     bm = __shfl(bm, 0, 64);
     const float mn = fmaxf(m, bm);
-    const float alpha = __builtin_amdgcn_exp2f(m - mn);  // m = -inf at first: exp2(-inf) = 0
+    const float mp = mn == -__builtin_inff() ? 0.0f : mn;  // no score above -inf yet: P = 0
+    const float alpha = __builtin_amdgcn_exp2f(m - mp);    // m = -inf at first: exp2(-inf) = 0
     m = mn;
-    const float p = lane < 16 ? __builtin_amdgcn_exp2f(s - m) : 0.0f;
+    const float p = lane < 16 ? __builtin_amdgcn_exp2f(s - mp) : 0.0f;
     l = l * alpha + p;
     if (lane < 16) pw[w][lane] = p;
     __builtin_amdgcn_wave_barrier();
