@@ -1013,6 +1013,28 @@ static void decode_group_split(int64_t bh, int64_t tiles, int64_t s_k, int& n_sp
   n_split = int(cdiv(s_k, c));
 }
 
+// Grouped decode (several query heads per kv head in one workgroup, on the
+// matrix cores) or one head per workgroup.  The grouped kernel reads the cache
+// once instead of once per head but is the longer chain for a workgroup.  So a
+// call that fills the GPU at most once with a 64-key workgroup per head and
+// has every head's reads served by the caches in a few microseconds goes head
+// by head: at most 512 workgroups (two per CU), below 16 MiB read in all (24
+// at D = 512, where the grouped kernel runs one wave per SIMD).  A single
+// 128-key split of the grouped kernel needs no merge launch: always grouped up
+// to D = 256.  us by head / grouped: 8 heads on 4 x 128, 128 keys 7.7 / 7.2,
+// 1000 keys 8.3 / 10.2, 4113 keys 12.7 / 11.4; 32 on 8 x 128, 1000 keys 10.0 /
+// 10.6, 4113 keys 23.1 / 14.7; 2 on 1 x 128, 4113 keys 8.6 / 10.3, 16384 keys
+// 12.9 / 11.8; 32 on 16 x 64, 1000 keys 8.2 / 9.1; 32 on 4 x 512, 128 keys
+// 22.2 / 29.3, 1000 keys 55.5 / 34.8.  Of 945 shapes (groups of 2 to 8, 100 to
+// 60000 keys) 22 are more than 3 % slower than the other kernel would be, by
+// 4 us at most; the grouped kernel alone would be at 234, by up to 50 %.
+static bool decode_grouped(int64_t bh, int64_t kv_group, int64_t s_k, int64_t D) {
+  if (kv_group == 1) return false;
+  if (D <= 256 && s_k <= 128) return true;
+  const int64_t bytes = 4 * D * bh * s_k;  // K and V, once per head
+  return bh * cdiv(s_k, 64) > 512 || bytes >= (int64_t(D > 256 ? 24 : 16) << 20);
+}
+
 size_t msa_decode_workspace_bytes(int64_t batch, int64_t heads, int64_t s_k, int32_t head_dim) {
   if (batch <= 0 || heads <= 0 || s_k <= 0 || head_dim <= 0) return 0;
   int ns, ch;
@@ -1058,8 +1080,11 @@ int msa_decode_attention(const msa_tensor4* q, const msa_tensor4* k, const msa_t
   dp.heads = int(H);
   dp.kv_group = int(H / Hkv);
   dp.s_k = int(Sk);
-  if (dp.kv_group == 1) decode_split(B * H, Sk, dp.n_split, dp.chunk);
-  else decode_group_split(B * H, B * Hkv * cdiv(dp.kv_group, 16), Sk, dp.n_split, dp.chunk);
+  dp.grouped = decode_grouped(B * H, dp.kv_group, Sk, D);
+  if (dp.grouped)
+    decode_group_split(B * H, B * Hkv * cdiv(dp.kv_group, 16), Sk, dp.n_split, dp.chunk);
+  else
+    decode_split(B * H, Sk, dp.n_split, dp.chunk);
   dp.scale_log2 = float(double(scale) * 1.4426950408889634);
   dp.part = static_cast<float*>(workspace);
   dp.ml = dp.part + B * H * dp.n_split * D;

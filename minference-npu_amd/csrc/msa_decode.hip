@@ -6,8 +6,9 @@
 // MInference-NPU/minference/modules/minference_forward.py:488-490.
 //
 // Bound by HBM: K and V are read once, 4*D bytes per key and kv head.  Two
-// kernels, chosen by the heads that share a kv head: decode_kernel (one head,
-// VALU) and decode_group_kernel (two or more, matrix cores).  Measured:
+// kernels: decode_kernel (a workgroup takes one head, VALU) and
+// decode_group_kernel (the heads of a kv head, matrix cores); decode_grouped in
+// msa_abi.hip has the line between them.  Measured:
 // 32 heads on 32 kv heads x 96, 65536 keys: 127.5 us VALU, 141 us matrix
 // cores (at D = 96 a quarter of its V lanes have no dims to read); 8 x 32
 // heads on 8 kv heads x 128, 16384 keys: 200.8 us VALU (every head reads its
@@ -28,7 +29,7 @@ namespace msa {
 #define INLINE __attribute__((always_inline))
 
 // ---------------------------------------------------------------------------
-// One query head per kv head: a GEMV pair (the matrix cores would idle on 15
+// One query head per workgroup: a GEMV pair (the matrix cores would idle on 15
 // of 16 rows), fp32 on the VALU.
 //
 // Split-K: the grid is (n_split, B*H); workgroup (s, b*H+h) walks keys
@@ -550,7 +551,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(DecodeParams P) {
 
 template <typename T, bool OUT_F32, int D>
 static hipError_t launch_decode_t(const DecodeParams& p, hipStream_t st) {
-  if (p.kv_group == 1) {
+  if (!p.grouped) {
     hipLaunchKernelGGL((decode_kernel<T, D>), dim3(p.n_split, p.batch * p.heads), dim3(256), 0, st,
                        p);
   } else {
@@ -560,7 +561,7 @@ static hipError_t launch_decode_t(const DecodeParams& p, hipStream_t st) {
                        p);
   }
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || (p.kv_group > 1 && p.n_split == 1)) return e;
+  if (e != hipSuccess || (p.grouped && p.n_split == 1)) return e;
   hipLaunchKernelGGL((decode_combine_kernel<T, OUT_F32, D>), dim3(p.batch * p.heads), dim3(256), 0,
                      st, p);
   return hipGetLastError();

@@ -213,6 +213,7 @@ struct DecodeParams {
   int64_t v_sb, v_sh, v_ss;
   int64_t o_sb, o_sh;
   int batch, heads, kv_group, s_k;
+  bool grouped;        // decode_group_kernel, else decode_kernel
   int n_split, chunk;  // key range of split s: [s*chunk, min((s+1)*chunk, s_k))
   float scale_log2;    // softmax scale * log2(e)
   float* part;         // workspace [batch*heads][n_split][D]: unnormalised O per split

@@ -59,6 +59,31 @@ def test_row_stride_and_late_maximum(gpu_device):
            boost=[(3, 3.0), (700, 8.0), (1500, 30.0), (1999, 60.0)])
 
 
+def _grouped_batch(H, S):
+    """The smallest batch that the grouped kernel takes at every length and
+    head dim: more than 512 64-key workgroups of one head each (smaller calls
+    may go head by head)."""
+    return 512 // (H * -(-S // 64)) + 1
+
+
+@pytest.mark.parametrize("S", [1, 33, 129, 160, 257, 500, 1025])
+@pytest.mark.parametrize("H,Hkv,D,dtype", [(8, 4, 64, torch.float16), (8, 2, 96, torch.bfloat16),
+                                           (17, 1, 128, torch.bfloat16),
+                                           (8, 2, 256, torch.float16), (4, 1, 512, torch.bfloat16)])
+def test_lengths_of_many_heads(gpu_device, S, H, Hkv, D, dtype):
+    _check(gpu_device, _grouped_batch(H, S), H, Hkv, S, D, dtype)
+
+
+# Either side of every line between the kernels: 128 keys, 512 workgroups of a
+# head, 16 MiB (24 at D = 512) read head by head.
+@pytest.mark.parametrize("B,H,Hkv,S,D", [
+    (1, 8, 4, 128, 128), (1, 8, 4, 129, 128), (1, 32, 8, 1024, 64), (1, 32, 8, 1025, 64),
+    (1, 2, 1, 16383, 128), (1, 2, 1, 16384, 128), (1, 4, 1, 3071, 512), (1, 4, 1, 3072, 512),
+    (1, 4, 1, 128, 512)])
+def test_either_kernel(gpu_device, B, H, Hkv, S, D):
+    _check(gpu_device, B, H, Hkv, S, D, torch.bfloat16)
+
+
 # Rows past the cache's end: the last 16- or 32-key block of a wave reaches
 # over S (by up to 31 rows), and those rows must read as zeros, whatever lies
 # there.  The rows past S are NaN here, where 0 * NaN would show.  (2, 2): the
@@ -72,8 +97,9 @@ def test_rows_past_the_cache_read_as_zeros(gpu_device, H, Hkv, S, D, dtype):
     from minference.backend.attention import decode_dense
 
     g = torch.Generator(gpu_device).manual_seed(S + D)
-    q = torch.randn(2, H, 1, D, device=gpu_device, generator=g).to(dtype)
-    k, v = (torch.randn(2, Hkv, S + 64, D, device=gpu_device, generator=g).to(dtype)
+    B = _grouped_batch(H, S) if H > Hkv else 2
+    q = torch.randn(B, H, 1, D, device=gpu_device, generator=g).to(dtype)
+    k, v = (torch.randn(B, Hkv, S + 64, D, device=gpu_device, generator=g).to(dtype)
             for _ in range(2))
     k[:, :, S:], v[:, :, S:] = float("nan"), float("nan")
     ks, vs = k[:, :, :S], v[:, :, :S]
@@ -94,9 +120,10 @@ def test_low_scores(gpu_device, H, Hkv, S, e):
 
     D = 64
     g = torch.Generator(gpu_device).manual_seed(S)
-    q = torch.zeros(1, H, 1, D, device=gpu_device, dtype=torch.bfloat16)
-    k = torch.zeros(1, Hkv, S, D, device=gpu_device, dtype=torch.bfloat16)
-    v = torch.randn(1, Hkv, S, D, device=gpu_device, generator=g).to(torch.bfloat16)
+    B = _grouped_batch(H, S) if H > Hkv else 1
+    q = torch.zeros(B, H, 1, D, device=gpu_device, dtype=torch.bfloat16)
+    k = torch.zeros(B, Hkv, S, D, device=gpu_device, dtype=torch.bfloat16)
+    v = torch.randn(B, Hkv, S, D, device=gpu_device, generator=g).to(torch.bfloat16)
     q[..., 5] = 2.0 ** e
     k[..., 5] = -(2.0 ** e)
     top = (7 * S) // 11
@@ -115,9 +142,10 @@ def test_infinite_scores(gpu_device, H, S):
 
     D = 64
     g = torch.Generator(gpu_device).manual_seed(3)
-    q = torch.randn(1, H, 1, D, device=gpu_device, generator=g).to(torch.bfloat16)
+    B = _grouped_batch(H, S) if H > 1 else 1
+    q = torch.randn(B, H, 1, D, device=gpu_device, generator=g).to(torch.bfloat16)
     q[..., 0] = 1.0
-    k, v = (torch.randn(1, 1, S, D, device=gpu_device, generator=g).to(torch.bfloat16)
+    k, v = (torch.randn(B, 1, S, D, device=gpu_device, generator=g).to(torch.bfloat16)
             for _ in range(2))
     low = torch.arange(S, device=gpu_device) % 40 != 17  # whole 16- and 32-key blocks among them
     k[:, :, low, 0] = -float("inf")
@@ -128,8 +156,8 @@ def test_infinite_scores(gpu_device, H, S):
     k[..., 0] = -float("inf")
     assert not decode_dense(q, k, v).any()
     # V: an infinite value reaches its own dim of every head and no other
-    k = torch.randn(1, 1, S, D, device=gpu_device, generator=g).to(torch.bfloat16)
-    v[0, 0, (7 * S) // 10, 9] = float("inf")
+    k = torch.randn(B, 1, S, D, device=gpu_device, generator=g).to(torch.bfloat16)
+    v[:, 0, (7 * S) // 10, 9] = float("inf")
     out = decode_dense(q, k, v)
     assert torch.isinf(out[..., 9]).all()
     assert torch.isfinite(out[..., :9]).all() and torch.isfinite(out[..., 10:]).all()
