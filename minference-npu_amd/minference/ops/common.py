@@ -75,20 +75,26 @@ def accepts_float32(names: Sequence[str], has_out: bool = True):
             # case the check fails (the host waits for the check only, so the
             # GPU never idles for it)
             flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
-            with torch.cuda.device(ts[0].device):
-                rounded = _abi.round_f32(ts, flag)
-                checked = torch.cuda.Event()
-                checked.record()
-            out = ba.arguments.get("out")
-            aliased = has_out and any(
-                out.untyped_storage().data_ptr() == t.untyped_storage().data_ptr() for t in ts)
-            if aliased:  # the op would write over what a second run reads
+            checked = torch.cuda.Event()
+            try:
+                with torch.cuda.device(ts[0].device):
+                    try:
+                        rounded = _abi.round_f32(ts, flag)
+                    finally:
+                        checked.record()
+                out = ba.arguments.get("out")
+                aliased = has_out and any(
+                    out.untyped_storage().data_ptr() == t.untyped_storage().data_ptr() for t in ts)
+                if aliased:  # the op would write over what a second run reads
+                    checked.synchronize()
+                    if int(flag[0]):
+                        rounded = [t.to(torch.bfloat16) for t in ts]
+                ba.arguments.update(zip(names, rounded))
+                result = fn(*ba.args, **ba.kwargs)
+            finally:
+                # the launch writes the flag through its address: nobody else
+                # may get that memory before it is done, raising ops included
                 checked.synchronize()
-                if int(flag[0]):
-                    rounded = [t.to(torch.bfloat16) for t in ts]
-            ba.arguments.update(zip(names, rounded))
-            result = fn(*ba.args, **ba.kwargs)
-            checked.synchronize()
             if int(flag[0]) and not aliased:
                 ba.arguments.update(zip(names, (t.to(torch.bfloat16) for t in ts)))
                 result = fn(*ba.args, **ba.kwargs)

@@ -75,3 +75,20 @@ def test_fp16_v_needs_no_scale_pass(gpu_device, dtype):
     assert torch.equal(fin, torch.isfinite(out))
     scale = v.double().abs().masked_fill(~torch.isfinite(v), 0).amax()
     assert float(((out - ref)[fin]).abs().max()) < 2e-3 * float(scale)
+
+
+def test_raising_op_waits_for_the_rounding(gpu_device):
+    """The launch writes the range flag through its address: an op that raises
+    (here: an output of the wrong shape) gives the call back only when the
+    launch is done with it."""
+    from minference import streaming_forward
+
+    q, k, v = (torch.randn(1, 2, 128, 64, device=gpu_device) for _ in range(3))
+    bad = torch.empty(1, 2, 127, 64, device=gpu_device)
+    with pytest.raises(ValueError):
+        streaming_forward(q, k, v, 16, 64, out=bad)
+    torch.cuda.synchronize()
+    torch.cuda._sleep(20_000_000)  # the rounding is queued behind some work
+    with pytest.raises(ValueError):
+        streaming_forward(q, k, v, 16, 64, out=bad)
+    assert torch.cuda.current_stream().query()
