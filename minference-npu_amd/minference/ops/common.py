@@ -34,6 +34,22 @@ def sixteen_bit_dtype(tensors: Sequence[torch.Tensor]) -> torch.dtype:
     return torch.float16
 
 
+def _long_op(ts: Sequence[torch.Tensor], causal: bool) -> bool:
+    """True when an op on float32 tensors [q, k, ...] waits for the range
+    check of their roundings before it is queued.  Waiting leaves the GPU idle
+    for 5 to 45 us of every call; not waiting costs a second run of the op when
+    a value lies beyond fp16's range.  The line is 2^37 operations of the
+    largest work the op can have, every visible pair (about 0.2 ms): causal
+    32 x 4096 x 96 streaming, below it, 126 us against 166 in range and 354
+    against 276 beyond it.  On the torch ops that other tensors take such calls
+    are slower in either case (487 and 570 us); at twice the line the longest
+    second runs no longer are (full attention 4 x 16384 x 64: 927 us run
+    twice, 834 on torch ops, 659 waiting)."""
+    q, k = ts[0], ts[1]
+    pairs = q.shape[2] * k.shape[2] / (2 if causal else 1)
+    return 4 * q.shape[0] * q.shape[1] * q.shape[3] * pairs >= 2 ** 37
+
+
 def accepts_float32(names: Sequence[str], has_out: bool = True):
     """Decorator for the public ops: called with float32 tensors ``names``,
     the op runs on their on-device roundings to sixteen_bit_dtype and, when
@@ -70,10 +86,14 @@ def accepts_float32(names: Sequence[str], has_out: bool = True):
                 dt = sixteen_bit_dtype(ts)
                 ba.arguments.update(zip(names, (t.to(dt) for t in ts)))
                 return fn(*ba.args, **ba.kwargs)
-            # fp16 roundings and the range check in one launch; the op is
-            # queued behind it and runs again on bf16 roundings in the rare
-            # case the check fails (the host waits for the check only, so the
-            # GPU never idles for it)
+            # fp16 roundings and the range check in one launch.  A short op is
+            # queued behind it, so the GPU does not idle while the host waits
+            # for the check, and runs again on bf16 roundings in the rare case
+            # the check fails; a long one, and one whose output overwrites an
+            # input, waits for the check first and runs once
+            out = ba.arguments.get("out")
+            wait = _long_op(ts, ba.arguments.get("causal", True)) or has_out and any(
+                out.untyped_storage().data_ptr() == t.untyped_storage().data_ptr() for t in ts)
             flag = torch.zeros(1, dtype=torch.int32, pin_memory=True)
             checked = torch.cuda.Event()
             try:
@@ -82,21 +102,20 @@ def accepts_float32(names: Sequence[str], has_out: bool = True):
                         rounded = _abi.round_f32(ts, flag)
                     finally:
                         checked.record()
-                out = ba.arguments.get("out")
-                aliased = has_out and any(
-                    out.untyped_storage().data_ptr() == t.untyped_storage().data_ptr() for t in ts)
-                if aliased:  # the op would write over what a second run reads
-                    checked.synchronize()
-                    if int(flag[0]):
-                        rounded = [t.to(torch.bfloat16) for t in ts]
                 ba.arguments.update(zip(names, rounded))
-                result = fn(*ba.args, **ba.kwargs)
+                del rounded
+                if not wait:
+                    result = fn(*ba.args, **ba.kwargs)
             finally:
                 # the launch writes the flag through its address: nobody else
                 # may get that memory before it is done, raising ops included
                 checked.synchronize()
-            if int(flag[0]) and not aliased:
-                ba.arguments.update(zip(names, (t.to(torch.bfloat16) for t in ts)))
+            again = int(flag[0]) != 0
+            if again:
+                for n, t in zip(names, ts):
+                    ba.arguments[n] = None  # the fp16 rounding makes room
+                    ba.arguments[n] = t.to(torch.bfloat16)
+            if wait or again:
                 result = fn(*ba.args, **ba.kwargs)
             return result
 

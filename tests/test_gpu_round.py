@@ -92,3 +92,27 @@ def test_raising_op_waits_for_the_rounding(gpu_device):
     with pytest.raises(ValueError):
         streaming_forward(q, k, v, 16, 64, out=bad)
     assert torch.cuda.current_stream().query()
+
+
+@pytest.mark.parametrize("big", [False, True])
+@pytest.mark.parametrize("S,causal", [(300, True), (32768, True), (32767, True), (23170, False),
+                                      (23171, False)])
+def test_long_op_runs_once(gpu_device, big, S, causal):
+    """From 2^37 operations on the op is queued when its type is known; below,
+    it may run a second time on bf16 roundings."""
+    from minference.ops.common import accepts_float32
+
+    seen = []
+
+    @accepts_float32(("q", "k", "v"))
+    def op(q, k, v, *, causal=True, out=None):
+        seen.append(q.dtype)
+        assert q.dtype == k.dtype == v.dtype and out.dtype == torch.float32
+        return out
+
+    q, k, v = (torch.zeros(1, 1, S, 64, device=gpu_device) for _ in range(3))
+    if big:
+        k[0, 0, S // 2, 3] = 7.0e4
+    op(q, k, v, causal=causal)
+    short = 4 * 64 * S * S // (2 if causal else 1) < 2 ** 37
+    assert seen == ([torch.float16, torch.bfloat16][0 if not big or short else 1:2 if big else 1])
