@@ -141,6 +141,9 @@ def block_sparse_attention_with_indices(
             "block_indices shape must be [B,H,n_q_blocks,topk_blocks]; "
             f"got {tuple(block_indices.shape)} for q={tuple(q.shape)} block_size={block_size}"
         )
+    # a block beyond both axes is block 0 alone at any size; the lists take 2^20 tokens
+    tile = _abi.MSA_BLOCK
+    bs = min(bs, math.ceil(max(S_q, k.shape[2]) / tile) * tile)
     return _attend_ids(q, k, v, block_indices.to(q.device), bs, out)
 
 

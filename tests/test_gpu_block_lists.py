@@ -42,3 +42,14 @@ def test_other_id_types(gpu_device):
         assert torch.equal(block_sparse_attention_with_indices(q, k, v, t), want)
     with pytest.raises(ValueError):
         block_sparse_attention_with_indices(q, k, v, ids[..., :0])
+
+
+@pytest.mark.parametrize("block", [320, 1 << 20, (1 << 20) + 64, 1 << 33])
+def test_block_beyond_the_keys(gpu_device, block):
+    """One block that holds every token, at any size: id 0 is causal attention."""
+    from minference.ops.block_sparse_kernel import block_sparse_attention_with_indices
+
+    q, k, v = (torch.randn(1, 2, 300, 96, device=gpu_device).bfloat16() for _ in range(3))
+    ids = torch.tensor([0, 1, -1, 0]).expand(1, 2, 1, 4)
+    want = block_sparse_attention_with_indices(q, k, v, torch.arange(5).expand(1, 2, 5, 5))
+    assert torch.equal(block_sparse_attention_with_indices(q, k, v, ids, block), want)
