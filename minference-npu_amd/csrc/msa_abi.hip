@@ -573,39 +573,94 @@ static double prefix_cost(const HeadWork& w, double m) {
   return tiles / w.div + w.fixed * m;
 }
 
+// attention workgroups that share a CU (not vertical_and_slash)
+static int wg_per_cu(int D) { return D > 128 ? 1 : 2; }
+
+// Contiguous item ranges of the 8 XCDs over n entries of nq query blocks each,
+// head-major, query blocks longest-first: XCD x takes items start[x] ..
+// start[x + 1] - 1.
+struct XcdRanges {
+  int start[9];
+};
+
+// cost of the first g items; cum[i]: cost of the entries before i
+static double items_cost(const double* cum, const HeadWork* work, int nq, int g) {
+  const int h = g / nq, r = g - h * nq;
+  return r ? cum[h] + prefix_cost(work[h], nq) - prefix_cost(work[h], nq - r) : cum[h];
+}
+
+// ranges of equal estimated cost
+static void ranges_by_cost(const double* cum, const HeadWork* work, int n, int nq, XcdRanges& rg) {
+  rg.start[0] = 0;
+  rg.start[8] = n * nq;
+  int h = 0;
+  for (int x = 1; x < 8; ++x) {
+    const double target = cum[n] * x / 8.0;
+    while (h < n - 1 && cum[h + 1] < target) ++h;
+    int lo = 0, hi = nq;  // first r items (bq = nq-1 .. nq-r) of head h cost >= need
+    while (lo < hi) {
+      const int mid = (lo + hi) / 2;
+      if (items_cost(cum, work, nq, h * nq + mid) >= target) hi = mid;
+      else lo = mid + 1;
+    }
+    rg.start[x] = std::max(rg.start[x - 1], h * nq + lo);
+  }
+}
+
+// Time of a launch of these ranges, in tiles of a workgroup that shares its
+// CU: whole rounds of an XCD's mean item, 0.6 for a last round whose items
+// have a CU each.
+static double ranges_time(const XcdRanges& rg, const double* cum, const HeadWork* work, int nq,
+                          int per_cu) {
+  const int cus = cus_per_xcd(), slots = cus * per_cu;
+  double worst = 0.0;
+  for (int x = 0; x < 8; ++x) {
+    const int a = rg.start[x], b = rg.start[x + 1], n = b - a;
+    if (n <= 0) continue;
+    const double sum = items_cost(cum, work, nq, b) - items_cost(cum, work, nq, a);
+    const int full = n / slots, rem = n % slots;
+    const double rounds = full + (rem == 0 ? 0.0 : per_cu == 2 && rem <= cus ? 0.6 : 1.0);
+    // 3: what an item's start and end take beyond HeadWork::fixed
+    const double mean = sum / n + 3.0;
+    double longest = 0.0;
+    for (int h = a / nq; h * nq < b; ++h)
+      longest = fmax(longest, work[h].longest(nq) / work[h].div);
+    worst = fmax(worst, fmax(mean * rounds, longest * (per_cu == 2 && n <= cus ? 0.6 : 1.0)));
+  }
+  return worst;
+}
+
 // Items of one launch: the listed entries ((batch, head) pairs or key splits
-// of one, AttnParams::head_order codes), head-major, query blocks
-// longest-first; the 8 XCDs (round-robin workgroup dispatch) take contiguous
-// ranges of equal estimated cost, so each XCD's L2 serves few heads and a
-// heavy head can be shared by two XCDs.
-static void order_items(AttnParams& ap, const int* entries, const HeadWork* work, int n) {
+// of one, AttnParams::head_order codes), head-major, so each XCD's L2 serves
+// few heads and a heavy head can be shared by two XCDs.  The 8 XCDs
+// (round-robin workgroup dispatch) take ranges of equal estimated cost, or
+// (per_cu workgroups on a CU; 0: never) of equal count where that is the
+// shorter launch: in one or two rounds an XCD with a few items more than the
+// others takes a round more, whatever they cost.  Chunks of 96-dim prompts, 10 % dense,
+// 60 % block and 30 % stream heads, by cost / by count: 32 heads, 1000 rows of
+// 5000 keys 110 / 91 us, 2000 of 5000 150 / 134; 8 heads, 2000 of 20000 91 /
+// 77; 4000 of 20000, many rounds of unequal items, 377 / 458.
+static void order_items(AttnParams& ap, const int* entries, const HeadWork* work, int n,
+                        int per_cu) {
   const int nq = ap.n_qb;
   ap.n_hl = n;
-  double head_tot[kMaxEntries], total = 0.0;
+  double cum[kMaxEntries + 1];
+  cum[0] = 0.0;
   for (int i = 0; i < n; ++i) {
     ap.head_order[i] = entries[i];
-    head_tot[i] = prefix_cost(work[i], nq);
-    total += head_tot[i];
+    cum[i + 1] = cum[i] + prefix_cost(work[i], nq);
   }
-  int prev = 0, h = 0;
-  double before = 0.0;  // cost of the heads before h
+  XcdRanges rg;
+  ranges_by_cost(cum, work, n, nq, rg);
+  if (per_cu > 0) {
+    XcdRanges even;
+    for (int x = 0; x <= 8; ++x) even.start[x] = int(int64_t(n) * nq * x / 8);
+    if (ranges_time(even, cum, work, nq, per_cu) < 0.97 * ranges_time(rg, cum, work, nq, per_cu))
+      rg = even;
+  }
   for (int x = 0; x < 8; ++x) {
-    int cut = n * nq;
-    if (x < 7) {
-      const double target = total * (x + 1) / 8.0;
-      while (h < n - 1 && before + head_tot[h] < target) before += head_tot[h++];
-      const double need = target - before;
-      int lo = 0, hi = nq;  // first r items (bq = nq-1 .. nq-r) of head h cost >= need
-      while (lo < hi) {
-        const int mid = (lo + hi) / 2;
-        if (prefix_cost(work[h], nq) - prefix_cost(work[h], nq - mid) >= need) hi = mid;
-        else lo = mid + 1;
-      }
-      cut = std::max(prev, h * nq + lo);
-    }
-    ap.xcd_start[x] = prev;
-    ap.xcd_count[x] = cut - prev;
-    prev = cut;
+    ap.xcd_start[x] = rg.start[x];
+    ap.xcd_count[x] = rg.start[x + 1] - rg.start[x];
   }
 }
 
@@ -668,7 +723,7 @@ static void plan_items(const msa_head_desc* heads, int H, int BH, int n_qb, int 
     total += prefix_cost(work[i], n_qb);
     longest = fmax(longest, work[i].longest(n_qb));
   }
-  const double slots = 8.0 * cus_per_xcd() * (D > 128 ? 1 : 2);
+  const double slots = 8.0 * cus_per_xcd() * wg_per_cu(D);
   const double piece = fmax(total / slots / 2.0, D < 128 ? 64.0 : 32.0);
   const double least = fmax(D < 128 ? 160.0 : 96.0, 1.5 * piece);
   int ns = 1, n_sp = 0;
@@ -838,7 +893,7 @@ static int layer_attention_impl(const msa_tensor4* q, const msa_tensor4* k, cons
   if (n_vs == 0) {
     if (BH <= kMaxHeads) {
       if (pl.n == 0) return MSA_OK;
-      order_items(ap, pl.entry, pl.work, pl.n);
+      order_items(ap, pl.entry, pl.work, pl.n, wg_per_cu(D));
       ap.n_split = pl.n_split;
       ap.part = static_cast<float*>(split_ws);
     } else {
@@ -935,11 +990,11 @@ static int layer_attention_impl(const msa_tensor4* q, const msa_tensor4* k, cons
   vp.vs_slots = vs->n_slots;
   vp.vs_cap = vl.cap;
   vp.nv_pad = vl.nv_pad;
-  order_items(vp, vs_pairs, vs_work, n_v);
+  order_items(vp, vs_pairs, vs_work, n_v, 0);  // its workgroups take items as they come
   e = launch_attention_vs(vp, q->dtype, o->dtype, D, hs);
   if (e != hipSuccess) return int(e);
   if (n_o) {
-    order_items(ap, other, other_work, n_o);
+    order_items(ap, other, other_work, n_o, wg_per_cu(D));
     e = launch_attention(ap, q->dtype, o->dtype, D, hs);
   }
   return e == hipSuccess ? MSA_OK : int(e);
