@@ -611,8 +611,8 @@ static void ranges_by_cost(const double* cum, const HeadWork* work, int n, int n
 // CU: whole rounds of an XCD's mean item, 0.6 for a last round whose items
 // have a CU each.
 static double ranges_time(const XcdRanges& rg, const double* cum, const HeadWork* work, int nq,
-                          int per_cu) {
-  const int cus = cus_per_xcd(), slots = cus * per_cu;
+                          int cus, int per_cu) {
+  const int slots = cus * per_cu;
   double worst = 0.0;
   for (int x = 0; x < 8; ++x) {
     const int a = rg.start[x], b = rg.start[x + 1], n = b - a;
@@ -630,34 +630,43 @@ static double ranges_time(const XcdRanges& rg, const double* cum, const HeadWork
   return worst;
 }
 
-// Items of one launch: the listed entries ((batch, head) pairs or key splits
-// of one, AttnParams::head_order codes), head-major, so each XCD's L2 serves
-// few heads and a heavy head can be shared by two XCDs.  The 8 XCDs
-// (round-robin workgroup dispatch) take ranges of equal estimated cost, or
-// (per_cu workgroups on a CU; 0: never) of equal count where that is the
-// shorter launch: in one or two rounds an XCD with a few items more than the
-// others takes a round more, whatever they cost.  Chunks of 96-dim prompts, 10 % dense,
-// 60 % block and 30 % stream heads, by cost / by count: 32 heads, 1000 rows of
-// 5000 keys 110 / 91 us, 2000 of 5000 150 / 134; 8 heads, 2000 of 20000 91 /
-// 77; 4000 of 20000, many rounds of unequal items, 377 / 458.
-static void order_items(AttnParams& ap, const int* entries, const HeadWork* work, int n,
-                        int per_cu) {
-  const int nq = ap.n_qb;
-  ap.n_hl = n;
+// Ranges of n entries: of equal estimated cost, or (per_cu workgroups on each
+// of an XCD's cus CUs; 0: never) of equal count where that is the shorter
+// launch: in one or two rounds an XCD with a few items more than the others
+// takes a round more, whatever they cost.  Not in a full prefill, whose short
+// first query blocks fill such a round up (2 heads x 8000 x 96: 61.5 us by
+// cost, 64.4 by count).  Returns the launch's estimated time (0 with per_cu =
+// 0).  Chunks of 96-dim prompts, 10 % dense, 60 % block and 30 % stream heads,
+// by cost / by count: 32 heads, 1000 rows of 5000 keys 110 / 91 us, 2000 of
+// 5000 150 / 134; 8 heads, 2000 of 20000 91 / 77; 32 heads, 4000 of 20000, many
+// rounds of unequal items, 377 / 458.
+static double pick_ranges(const HeadWork* work, int n, int nq, int cus, int per_cu,
+                          XcdRanges& rg) {
   double cum[kMaxEntries + 1];
   cum[0] = 0.0;
-  for (int i = 0; i < n; ++i) {
-    ap.head_order[i] = entries[i];
-    cum[i + 1] = cum[i] + prefix_cost(work[i], nq);
-  }
-  XcdRanges rg;
+  for (int i = 0; i < n; ++i) cum[i + 1] = cum[i] + prefix_cost(work[i], nq);
   ranges_by_cost(cum, work, n, nq, rg);
-  if (per_cu > 0) {
-    XcdRanges even;
-    for (int x = 0; x <= 8; ++x) even.start[x] = int(int64_t(n) * nq * x / 8);
-    if (ranges_time(even, cum, work, nq, per_cu) < 0.97 * ranges_time(rg, cum, work, nq, per_cu))
-      rg = even;
-  }
+  if (per_cu == 0) return 0.0;
+  const double by_cost = ranges_time(rg, cum, work, nq, cus, per_cu);
+  if (work[0].off == 0.0) return by_cost;
+  XcdRanges even;
+  for (int x = 0; x <= 8; ++x) even.start[x] = int(int64_t(n) * nq * x / 8);
+  const double by_count = ranges_time(even, cum, work, nq, cus, per_cu);
+  if (by_count >= 0.97 * by_cost) return by_cost;
+  rg = even;
+  return by_count;
+}
+
+// Items of one launch: the listed entries ((batch, head) pairs or key splits
+// of one, AttnParams::head_order codes), head-major, the 8 XCDs (round-robin
+// workgroup dispatch) taking contiguous ranges, so each XCD's L2 serves few
+// heads and a heavy head can be shared by two XCDs.
+static void order_items(AttnParams& ap, const int* entries, const HeadWork* work, int n,
+                        int per_cu) {
+  ap.n_hl = n;
+  for (int i = 0; i < n; ++i) ap.head_order[i] = entries[i];
+  XcdRanges rg;
+  pick_ranges(work, n, ap.n_qb, ap.wg_per_xcd, per_cu, rg);
   for (int x = 0; x < 8; ++x) {
     ap.xcd_start[x] = rg.start[x];
     ap.xcd_count[x] = rg.start[x + 1] - rg.start[x];
@@ -685,30 +694,46 @@ static void interleave_kinds(int* list, int n, const msa_head_desc* heads, int H
 // pair but the skipped ones, and the key splits.
 struct ItemPlan {
   int n = 0;                 // entries
-  int n_split = 1, n_sp = 0;  // splits per split pair, split pairs
+  int n_sp = 0, n_rows = 0;  // split pairs, key splits of all of them
   int entry[kMaxEntries];
   HeadWork work[kMaxEntries];
-  uint8_t pair[kMaxHeads];   // of each split pair
+  uint8_t pair[kMaxHeads], first[kMaxHeads], n_split[kMaxHeads];  // of each split pair
   // floats of the partial outputs
   size_t part_floats(int n_qb, int D) const {
-    return size_t(n_sp) * n_split * n_qb * MSA_BLOCK * (size_t(D) + 2);
+    return size_t(n_rows) * n_qb * MSA_BLOCK * (size_t(D) + 2);
+  }
+  // adds a pair in ns key splits (1: whole)
+  void add(int p, HeadWork w, int ns) {
+    w.div = ns;
+    if (ns > 1) {
+      pair[n_sp] = uint8_t(p);
+      first[n_sp] = uint8_t(n_rows);
+      n_split[n_sp++] = uint8_t(ns);
+    }
+    for (int k = 0; k < ns; ++k) {
+      entry[n] = ns == 1 ? p : int(0x80000000u | uint32_t(ns) << 20 | uint32_t(k) << 16 |
+                                   uint32_t(n_rows++) << 8 | uint32_t(p));
+      work[n++] = w;
+    }
   }
 };
 
 // Key splits: an item is one workgroup, so a launch takes at least as long as
 // its longest item.  Where that is well above the average load of the
 // workgroups the GPU holds at once (a chunk of a prompt against a long cache),
-// the long heads are cut into up to kMaxSplit key splits whose partial outputs
-// a second launch merges.  The piece aimed at is half the average load, and
-// not below 64 tiles; heads below 160 tiles stay whole: a piece writes 25 to
-// 64 KB that the merge (5 to 8 us) reads again, more than shorter heads gain
-// (4 dense heads x 6000 x 96, 94 tiles: 50 us whole, 59 in pieces of 24).  At
-// D >= 128 a tile takes about twice as long, so the lines lie at 32 and 96
-// (300 rows of 20000 keys, 32 heads on 8 x 128, 100 tiles: 101 us whole, 93
-// in pieces of 32; D = 64: 83.4 whole, 84.8).
-// 2000 rows of 30000 keys, 32 heads, 30 % stream / 60 % block / 10 % dense,
-// whole layer: D = 96 407 -> 320 us, D = 128 476 -> 363 us; 100 rows of 40000
-// keys: 427 -> 193 us.
+// the long heads are cut into up to kMaxSplit key splits each, whose partial
+// outputs a second launch merges.  The piece aimed at is half the average
+// load, and not below 64 tiles (32 at D >= 128, where a tile takes about twice
+// as long); heads below 160 (64) tiles stay whole: a piece writes 25 to 64 KB
+// that the merge reads again, more than shorter heads gain (4 dense heads x
+// 6000 x 96, 94 tiles: 50 us whole, 59 in pieces of 24).  Splitting a launch
+// that fills its rounds gains nothing, so the split plan is taken only where
+// its estimated time and the merge's, about 10 tiles, stay below the whole
+// one's.  D = 96, whole / in 2 to 4 splits: 32 dense heads, 1000 rows of 20000
+// keys (512 items, one round) 307 / 346 us; 300 rows of 20000 (160 items) 212
+// / 171; 8 dense heads, 1000 of 40000 263 / 160.  D = 128, 32 heads of 50 %
+// block, 50 % stream on 8, 1000 rows of 40000 keys (512 items of 66 to 100
+// tiles) 173 / 211; 300 of 5000 (160 items) 86 / 71.
 static void plan_items(const msa_head_desc* heads, int H, int BH, int n_qb, int n_kb, int topk_max,
                        int D, bool split, ItemPlan& pl) {
   int pairs[kMaxHeads];
@@ -723,31 +748,30 @@ static void plan_items(const msa_head_desc* heads, int H, int BH, int n_qb, int 
     total += prefix_cost(work[i], n_qb);
     longest = fmax(longest, work[i].longest(n_qb));
   }
-  const double slots = 8.0 * cus_per_xcd() * wg_per_cu(D);
+  const int cus = cus_per_xcd(), per_cu = wg_per_cu(D);
+  const double slots = 8.0 * cus * per_cu;
   const double piece = fmax(total / slots / 2.0, D < 128 ? 64.0 : 32.0);
-  const double least = fmax(D < 128 ? 160.0 : 96.0, 1.5 * piece);
-  int ns = 1, n_sp = 0;
+  const double least = fmax(D < 128 ? 160.0 : 64.0, 1.5 * piece);
+  pl = ItemPlan();
   if (split && D <= 256 && longest > least) {
-    ns = int(fmin(double(kMaxSplit), ceil(longest / piece)));
-    for (int i = 0; i < n; ++i) n_sp += work[i].longest(n_qb) > least;
-    while (ns > 1 && n + (ns - 1) * n_sp > kMaxEntries) --ns;
-  }
-  pl.n = 0;
-  pl.n_sp = 0;
-  pl.n_split = ns;
-  for (int i = 0; i < n; ++i) {
-    if (ns == 1 || work[i].longest(n_qb) <= least) {
-      pl.entry[pl.n] = pairs[i];
-      pl.work[pl.n++] = work[i];
-      continue;
+    for (int most = kMaxSplit; most > 1; --most) {
+      int ns[kMaxHeads], entries = 0;
+      for (int i = 0; i < n; ++i) {
+        const double len = work[i].longest(n_qb);
+        ns[i] = len > least ? std::min(most, int(ceil(len / piece))) : 1;
+        entries += ns[i];
+      }
+      if (entries > kMaxEntries) continue;
+      for (int i = 0; i < n; ++i) pl.add(pairs[i], work[i], ns[i]);
+      break;
     }
-    work[i].div = ns;
-    for (int k = 0; k < ns; ++k) {
-      pl.entry[pl.n] = int(0x80000000u | uint32_t(k) << 16 | uint32_t(pl.n_sp) << 8 | uint32_t(pairs[i]));
-      pl.work[pl.n++] = work[i];
-    }
-    pl.pair[pl.n_sp++] = uint8_t(pairs[i]);
+    XcdRanges rg;
+    if (pl.n_sp && pick_ranges(pl.work, pl.n, n_qb, cus, per_cu, rg) + 10.0 <
+                       pick_ranges(work, n, n_qb, cus, per_cu, rg))
+      return;
+    pl = ItemPlan();
   }
+  for (int i = 0; i < n; ++i) pl.add(pairs[i], work[i], 1);
 }
 
 size_t msa_split_workspace_bytes(const msa_tensor4* q, const msa_tensor4* k,
@@ -894,7 +918,6 @@ static int layer_attention_impl(const msa_tensor4* q, const msa_tensor4* k, cons
     if (BH <= kMaxHeads) {
       if (pl.n == 0) return MSA_OK;
       order_items(ap, pl.entry, pl.work, pl.n, wg_per_cu(D));
-      ap.n_split = pl.n_split;
       ap.part = static_cast<float*>(split_ws);
     } else {
       ap.n_hl = 0;  // every pair, plain order
@@ -909,9 +932,10 @@ static int layer_attention_impl(const msa_tensor4* q, const msa_tensor4* k, cons
       cp.heads = ap.heads;
       cp.s_q = ap.s_q;
       cp.n_qb = n_qb;
-      cp.n_split = pl.n_split;
       cp.n_pairs = pl.n_sp;
-      memcpy(cp.pair, pl.pair, sizeof(cp.pair));
+      memcpy(cp.pair, pl.pair, pl.n_sp);
+      memcpy(cp.first, pl.first, pl.n_sp);
+      memcpy(cp.n_split, pl.n_split, pl.n_sp);
       e = launch_combine(cp, q->dtype, o->dtype, D, hs);
     }
     return e == hipSuccess ? MSA_OK : int(e);

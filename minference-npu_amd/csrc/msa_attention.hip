@@ -480,6 +480,7 @@ __device__ inline void item_tiles(const AttnParams& P, int kind, int64_t list_ro
 struct Item {
   int hh, bq;
   int split;     // -1: the whole item
+  int n_split;
   int part_row;  // row of AttnParams::part
 };
 
@@ -487,6 +488,7 @@ struct Item {
 __device__ inline bool find_item(const AttnParams& P, Item& it) {
   const int xcd = blockIdx.x & 7;
   it.split = -1;
+  it.n_split = 1;
   it.part_row = 0;
   if (P.n_hl) {
     const int r = int(blockIdx.x) >> 3;
@@ -497,8 +499,9 @@ __device__ inline bool find_item(const AttnParams& P, Item& it) {
     it.hh = e & 0xff;
     it.bq = P.n_qb - 1 - (g - hl * P.n_qb);
     if (e < 0) {
-      it.split = (e >> 16) & 0xff;
-      it.part_row = (((e >> 8) & 0xff) * P.n_split + it.split) * P.n_qb + it.bq;
+      it.split = (e >> 16) & 15;
+      it.n_split = (e >> 20) & 15;
+      it.part_row = ((e >> 8) & 0xff) * P.n_qb + it.bq;
     }
   } else {
     // plain order: every (batch, head) pair; the host lists no item of a
@@ -655,7 +658,7 @@ void attn_kernel(AttnParams P) {
   bool is_full = false, is_stream = false;
   const int skm1 = P.s_k - 1;
 
-  auto init_item = [&](const int hh, const int bq, const int split) INLINE {
+  auto init_item = [&](const int hh, const int bq, const int split, const int n_split) INLINE {
     b = hh / P.heads;
     h = hh - b * P.heads;
     const int kvh = h / P.kv_group;
@@ -682,7 +685,7 @@ void attn_kernel(AttnParams P) {
       item_tiles(P, kind, (int64_t(b) * P.idx_slots + hd_slot) * P.n_qb + bq, a0, a1, n_init,
                  n_local, seq);
       if (split >= 0)
-        seq.narrow(seq.total * split / P.n_split, seq.total * (split + 1) / P.n_split);
+        seq.narrow(seq.total * split / n_split, seq.total * (split + 1) / n_split);
     }
     total = seq.total;
     mpos = max(min(seq.mpos, total), 0);
@@ -1140,7 +1143,7 @@ void attn_kernel(AttnParams P) {
       __syncthreads();
       if (g < 0) break;
       const int hl = g / P.n_qb;
-      init_item(int(P.head_order[hl]), P.n_qb - 1 - (g - hl * P.n_qb), -1);
+      init_item(int(P.head_order[hl]), P.n_qb - 1 - (g - hl * P.n_qb), -1, 1);
       load_q();
       reset_acc();
       start_tiles();
@@ -1150,7 +1153,7 @@ void attn_kernel(AttnParams P) {
   } else {
     Item it;
     if (!find_item(P, it)) return;
-    init_item(it.hh, it.bq, it.split);
+    init_item(it.hh, it.bq, it.split, it.n_split);
     load_q();
     reset_acc();
     start_tiles();
@@ -1224,7 +1227,7 @@ void attn_split_kernel(AttnParams P) {
   item_tiles(P, kind, (int64_t(b) * P.idx_slots + P.hd[h].slot) * P.n_qb + bq, a0, a0 + nrows - 1,
              n_init, n_local, seq);
   if (it.split >= 0)
-    seq.narrow(seq.total * it.split / P.n_split, seq.total * (it.split + 1) / P.n_split);
+    seq.narrow(seq.total * it.split / it.n_split, seq.total * (it.split + 1) / it.n_split);
   const int total = seq.total;
   const int mpos = max(min(seq.mpos, total), 0);
   const int64_t bk = int64_t(b) * (P.heads / P.kv_group) + kvh;
@@ -1756,7 +1759,7 @@ void attn_wide_kernel(AttnParams P) {
 
 // Merge of the key splits of an item: O = sum_s w_s O_s, w_s = l_s 2^(m_s - M)
 // over their sum.  Four workgroups per (split pair, query block), 16 rows
-// each, thread = 4 dims of a row at a time; 4 * n_split * D bytes read per
+// each, thread = 4 dims of a row at a time; 4 D bytes read per split and
 // row, bound by latency.
 template <typename T, bool OUT_F32, int D>
 __global__ __launch_bounds__(256) void attn_combine_kernel(CombineParams P) {
@@ -1765,14 +1768,15 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(CombineParams P) {
   __shared__ float wt[kMaxSplit][ROWS];
   const int item = int(blockIdx.x) >> 2, r0 = (int(blockIdx.x) & 3) * ROWS;
   const int sp = item / P.n_qb, bq = item - sp * P.n_qb;
+  const int ns = P.n_split[sp];
   const int64_t stride = int64_t(P.n_qb) * (kBlock * (D + 2));  // between splits
-  const float* part = P.part + (int64_t(sp) * P.n_split * P.n_qb + bq) * (kBlock * (D + 2));
+  const float* part = P.part + (int64_t(P.first[sp]) * P.n_qb + bq) * (kBlock * (D + 2));
   const int tid = threadIdx.x;
   if (tid < ROWS) {
     float m[kMaxSplit], l[kMaxSplit], M = -__builtin_inff(), L = 0.0f;
 #pragma unroll
     for (int s = 0; s < kMaxSplit; ++s) {
-      const float2 x = s < P.n_split
+      const float2 x = s < ns
                            ? *reinterpret_cast<const float2*>(part + s * stride + kBlock * D + 2 * (r0 + tid))
                            : make_float2(-1e30f, 0.0f);
       m[s] = x.x;
@@ -1796,7 +1800,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(CombineParams P) {
     const int ri = i / TPR, d = 4 * (i - ri * TPR);
     const int r = r0 + ri;
     float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int s = 0; s < P.n_split; ++s) {
+    for (int s = 0; s < ns; ++s) {
       const float4 x = *reinterpret_cast<const float4*>(part + s * stride + r * D + d);
       const float f = wt[s][ri];
       acc.x = __builtin_fmaf(f, x.x, acc.x);

@@ -77,8 +77,9 @@ struct CombineParams {
   const float* part;
   void* o;
   int64_t o_sb, o_sh, o_ss;
-  int heads, s_q, n_qb, n_split, n_pairs;
-  uint8_t pair[kMaxHeads];  // (batch, head) of each split pair
+  int heads, s_q, n_qb, n_pairs;
+  // of each split pair: (batch, head), first row group in `part`, key splits
+  uint8_t pair[kMaxHeads], first[kMaxHeads], n_split[kMaxHeads];
 };
 
 struct AttnParams {
@@ -102,13 +103,12 @@ struct AttnParams {
   // longest-first; XCD x (workgroup i with i % 8 == x) takes items
   // xcd_start[x] + (i / 8) for i / 8 < xcd_count[x].  An entry is a (batch,
   // head) pair (bits 0-7) or one key split of it (bit 31 set, bits 8-15: its
-  // index among the split pairs, bits 16-23: the split): the split takes its
-  // share of n_split of every query block's tiles and leaves the partial
+  // row group in `part`, bits 16-19: which split, bits 20-23: of how many): the
+  // split takes its share of every query block's tiles and leaves the partial
   // output in `part`.  n_hl == 0: every (batch, head) pair of the layer in
   // plain order.
   int n_hl;
-  int n_split;
-  float* part;  // [split pair][split][query block]: 64 x D floats, 64 (m, l)
+  float* part;  // [row group][query block]: 64 x D floats, 64 (m, l)
   int xcd_start[8];
   int xcd_count[8];
   int* queue;      // 8 counters of the XCD ranges (zeroed before each launch)
