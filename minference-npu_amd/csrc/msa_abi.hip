@@ -250,9 +250,10 @@ int msa_block_estimate_ex(const msa_tensor4* q, const msa_tensor4* k, const int3
 }
 
 // Attention workspace: staged V operands (fp16), staged K operands (input
-// dtype; written only where the attention kernel cannot read K in place,
-// see k_in_place), per-tile V maxima (fp32), per-head V exponents (int32),
-// then the work-queue counters of the attention launch.
+// dtype; written where the attention kernel does not read K in place, see
+// stage_k_mode), per-tile V maxima (fp32), per-head V exponents (int32), then
+// the work-queue counters of the attention launch and the flag that tells it
+// where K is.
 struct AttnLayout {
   size_t vt, kt, tmax, vexp, total;
 };
@@ -319,27 +320,33 @@ static bool k_stride_slow(const msa_tensor4* k) { return k->stride[2] % 64 != 32
 // what msa_stage_kv and every full prefill (S_q == S_k) leave in place
 static bool k_in_place(const msa_tensor4* k) { return k_can_stay(k) && !k_stride_slow(k); }
 
-// Staging K pays where enough query blocks read it: with few (a chunk of a
-// prompt against a long cache) the copy costs more than the loads it speeds
-// up.  A K tile's copy takes about 6.5 ns of the GPU at D = 128, a staged
-// tile's loads save about 60 ns of one CU: 27 uses.  The line is drawn at 32
-// (query blocks x query heads per kv head), for S_q < S_k only: in a full
-// prefill of that size K is a few MB.  (2000 rows of 30000 keys, 32 heads on
-// 8 x 128, 128 uses at most: whole layer 476 us staged, 489 in place.)
-static bool k_used_enough(const msa_tensor4* q, const msa_tensor4* k) {
-  return q->size[2] == k->size[2] ||
-         cdiv(q->size[2], MSA_BLOCK) * (q->size[1] / k->size[1]) >= 32;
+// Staging K pays where its tiles are read often enough: the copy takes about
+// 6.5 ns of the GPU a tile at D = 128, and below the line it costs more than
+// the loads it speeds up.  reads: tiles read by the launch's query blocks per
+// tile of K.  Measured over chunks of 64 to 4000 rows of 5000 to 40000 keys,
+// 4 to 32 heads, groups of 1 and 4, in place / staged: D = 64, 17 reads 262 /
+// 274 us, 21 375 / 353, 31 832 / 816; D = 128, 8 reads 570 / 621, 14 873 / 884
+// and 277 / 257, 16 927 / 896, 28 455 / 399.
+static double k_reads_needed(int64_t D) { return D < 128 ? 28.0 : 12.0; }
+constexpr double kAllReads = 1e30;  // a full prefill: K of that size is a few MB
+
+// reads of a chunk's layer before its heads are known: those of sparse heads,
+// taken as 100 tiles a query block (top-k 100, or a window of 4096 keys and
+// sinks, 66)
+static double k_reads_sparse(const msa_tensor4* q, const msa_tensor4* k) {
+  if (q->size[2] == k->size[2]) return kAllReads;
+  return double(cdiv(q->size[2], MSA_BLOCK)) * double(q->size[1] / k->size[1]) *
+         fmin(1.0, 100.0 / double(cdiv(k->size[2], MSA_BLOCK)));
 }
 
-// q: the query tensor where the caller has it (null: K staged by its stride
-// alone).  The choice travels to the attention launch in the workspace.
-static int stage_k_mode(const msa_tensor4* q, const msa_tensor4* k) {
+// The choice travels to the attention launch in the workspace.
+static int stage_k_mode(const msa_tensor4* k, double reads) {
   if (!k_can_stay(k)) return 1;
-  return k_stride_slow(k) && (!q || k_used_enough(q, k)) ? 1 : 0;
+  return k_stride_slow(k) && reads >= k_reads_needed(k->size[3]) ? 1 : 0;
 }
 
-static int stage_setup(const msa_tensor4* q, const msa_tensor4* k, const msa_tensor4* v,
-                       void* workspace, size_t workspace_bytes, StageParams& sp) {
+static int stage_setup(const msa_tensor4* k, const msa_tensor4* v, double k_reads, void* workspace,
+                       size_t workspace_bytes, StageParams& sp) {
   if (!k || !v || !k->data || !v->data) return MSA_E_NULL;
   for (int i = 0; i < 4; ++i) {
     if (v->size[i] <= 0) return MSA_E_RANK;
@@ -370,7 +377,7 @@ static int stage_setup(const msa_tensor4* q, const msa_tensor4* k, const msa_ten
   sp.kv_heads = int(Hkv);
   sp.s_k = int(Sk);
   sp.s_pad = int(cdiv(Sk, MSA_BLOCK) * MSA_BLOCK);
-  sp.stage_k = stage_k_mode(q, k);
+  sp.stage_k = stage_k_mode(k, k_reads);
   sp.k_flag = k_flag_of(workspace, need);
   return MSA_OK;
 }
@@ -384,7 +391,7 @@ static int stage_launch(const StageParams& sp, int dtype, int D, hipStream_t hs)
 int msa_stage_kv(const msa_tensor4* k, const msa_tensor4* v, void* workspace,
                  size_t workspace_bytes, msa_stream_t stream) {
   StageParams sp;
-  const int st = stage_setup(nullptr, k, v, workspace, workspace_bytes, sp);
+  const int st = stage_setup(k, v, kAllReads, workspace, workspace_bytes, sp);
   if (st != MSA_OK) return st;
   return stage_launch(sp, v->dtype, int(v->size[3]), reinterpret_cast<hipStream_t>(stream));
 }
@@ -394,7 +401,7 @@ int msa_stage_kv_pool(const msa_tensor4* q, const msa_tensor4* k, const msa_tens
                       size_t est_workspace_bytes, void* workspace, size_t workspace_bytes,
                       msa_stream_t stream) {
   StageParams sp;
-  int st = stage_setup(nullptr, k, v, workspace, workspace_bytes, sp);
+  int st = stage_setup(k, v, kAllReads, workspace, workspace_bytes, sp);
   if (st != MSA_OK) return st;
   if (n_slots > 0) {
     int16_t slot_kvp[kMaxHeads];
@@ -403,7 +410,7 @@ int msa_stage_kv_pool(const msa_tensor4* q, const msa_tensor4* k, const msa_tens
                     slot_kvp, L);
     if (st != MSA_OK) return st;
     sp.n_pool_wg = pool_workgroups(sp.pool);
-    sp.stage_k = stage_k_mode(q, k);
+    sp.stage_k = stage_k_mode(k, k_reads_sparse(q, k));
   } else if (n_slots < 0) {
     return MSA_E_HEADS;
   }
@@ -571,6 +578,21 @@ static double prefix_cost(const HeadWork& w, double m) {
     tiles = up * a + up * (up + 1) / 2 + (m - up) * k;
   }
   return tiles / w.div + w.fixed * m;
+}
+
+// reads of K (k_reads_sparse) by the heads of a layer
+static double k_reads(const msa_tensor4* q, const msa_tensor4* k, const msa_head_desc* heads,
+                      int topk_max) {
+  if (q->size[2] == k->size[2]) return kAllReads;
+  const int n_qb = int(cdiv(q->size[2], MSA_BLOCK)), n_kb = int(cdiv(k->size[2], MSA_BLOCK));
+  double tiles = 0.0;
+  for (int h = 0; h < int(q->size[1]); ++h) {
+    if (heads[h].kind == MSA_KIND_SKIP) continue;
+    HeadWork w = head_work(heads[h], n_qb, n_kb, topk_max);
+    w.fixed = 0.0;
+    tiles += prefix_cost(w, n_qb);
+  }
+  return tiles / (double(n_kb) * double(k->size[1]));
 }
 
 // attention workgroups that share a CU (not vertical_and_slash)
@@ -871,7 +893,7 @@ static int layer_attention_impl(const msa_tensor4* q, const msa_tensor4* k, cons
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
   if (stage) {
     StageParams sp;
-    st = stage_setup(q, k, v, workspace, workspace_bytes, sp);
+    st = stage_setup(k, v, k_reads(q, k, heads, topk_max), workspace, workspace_bytes, sp);
     if (st == MSA_OK) st = stage_launch(sp, v->dtype, D, hs);
     if (st != MSA_OK) return st;
   }
@@ -999,7 +1021,7 @@ static int layer_attention_impl(const msa_tensor4* q, const msa_tensor4* k, cons
     // the vertical_and_slash kernel reads staged K: stage the K the plain
     // staging left in place (V and its exponents are staged already)
     StageParams kp;
-    st = stage_setup(nullptr, k, v, workspace, workspace_bytes, kp);
+    st = stage_setup(k, v, kAllReads, workspace, workspace_bytes, kp);
     if (st != MSA_OK) return st;
     kp.stage_k = 2;
     kp.k_flag = nullptr;  // the other heads' launch still reads K in place

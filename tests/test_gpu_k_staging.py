@@ -1,0 +1,65 @@
+"""Which calls stage K: the staged half of the workspace stays untouched where
+the attention kernel reads K in place.  K is staged for a slow row stride (not
+an odd multiple of 64 bytes) where the launch reads each tile often enough:
+28 times at head dims below 128, 12 from 128 on, always in a full prefill."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _tensors(dev, H, Hkv, S_q, S_k, D, pad=0):
+    q = torch.randn(1, H, S_q, D, device=dev).bfloat16()
+    k = torch.randn(1, Hkv, S_k, D + pad, device=dev).bfloat16()[..., :D]
+    v = torch.randn(1, Hkv, S_k, D, device=dev).bfloat16()
+    return q, k, v
+
+
+def _staged(k, ws):
+    half = k.shape[0] * k.shape[1] * k.shape[3] * (-(-k.shape[2] // 64) * 64) * 2
+    kt = ws[half:2 * half]
+    return not bool((kt == 0x5A).all())
+
+
+@pytest.mark.parametrize("H,Hkv,S_q,S_k,D,pad,staged", [
+    (2, 2, 1000, 10000, 128, 0, True),     # 15 reads
+    (2, 2, 1000, 10000, 64, 0, False),
+    (2, 2, 2000, 10000, 64, 0, True),      # 29
+    (2, 2, 700, 10000, 128, 0, False),     # 11
+    (8, 2, 300, 10000, 128, 0, True),      # 20: 5 query blocks, groups of 4
+    (2, 2, 2000, 10000, 64, 32, False),    # a fast stride
+    (2, 2, 300, 300, 64, 0, True),         # full prefill
+])
+def test_dense(gpu_device, H, Hkv, S_q, S_k, D, pad, staged):
+    from minference import _abi
+
+    q, k, v = _tensors(gpu_device, H, Hkv, S_q, S_k, D, pad)
+    ws = _abi.workspace(_abi.attention_workspace_bytes(1, Hkv, S_k, D), gpu_device).fill_(0x5A)
+    out = torch.empty_like(q)
+    _abi.layer_attention(q, k, v, out, [(_abi.MSA_KIND_DENSE, 0, 0, -1, D ** -0.5)] * H, ws=ws)
+    assert _staged(k, ws) == staged
+    ref = torch.nn.functional.scaled_dot_product_attention(
+        q.float().cpu(), k.float().cpu().repeat_interleave(H // Hkv, 1),
+        v.float().cpu().repeat_interleave(H // Hkv, 1),
+        attn_mask=torch.ones(S_q, S_k, dtype=torch.bool).tril(S_k - S_q))
+    assert float((out.float().cpu() - ref).abs().max()) < 2e-2  # bf16 output below 4
+
+
+@pytest.mark.parametrize("H,Hkv,S_q,S_k,D,staged", [
+    (4, 4, 2000, 40000, 64, False),     # 32 query blocks of about 100 of 625 tiles: 5 reads
+    (4, 4, 2000, 40000, 128, False),
+    (16, 4, 2000, 20000, 128, True),    # 41
+    (4, 4, 4000, 10000, 64, True),      # 40
+    (4, 4, 700, 700, 64, True),
+])
+def test_sparse_layer(gpu_device, H, Hkv, S_q, S_k, D, staged):
+    from minference import _abi
+
+    q, k, v = _tensors(gpu_device, H, Hkv, S_q, S_k, D)
+    ws = _abi.workspace(_abi.attention_workspace_bytes(1, Hkv, S_k, D), gpu_device).fill_(0x5A)
+    est = _abi.workspace(_abi.estimate_workspace_bytes(1, 2, S_q, S_k, D), gpu_device)
+    _abi.stage_kv_pool(q, k, v, [0, 1], est, ws)
+    assert _staged(k, ws) == staged
