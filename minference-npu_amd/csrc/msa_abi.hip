@@ -720,6 +720,7 @@ struct ItemPlan {
   int entry[kMaxEntries];
   HeadWork work[kMaxEntries];
   uint8_t pair[kMaxHeads], first[kMaxHeads], n_split[kMaxHeads];  // of each split pair
+  void clear() { n = n_sp = n_rows = 0; }
   // floats of the partial outputs
   size_t part_floats(int n_qb, int D) const {
     return size_t(n_rows) * n_qb * MSA_BLOCK * (size_t(D) + 2);
@@ -746,9 +747,11 @@ struct ItemPlan {
 // the long heads are cut into up to kMaxSplit key splits each, whose partial
 // outputs a second launch merges.  The piece aimed at is half the average
 // load, and not below 64 tiles (32 at D >= 128, where a tile takes about twice
-// as long); heads below 160 (64) tiles stay whole: a piece writes 25 to 64 KB
-// that the merge reads again, more than shorter heads gain (4 dense heads x
-// 6000 x 96, 94 tiles: 50 us whole, 59 in pieces of 24).  Splitting a launch
+// as long); heads of up to 160 tiles (64 at D >= 128, 96 where the whole items
+// have a CU each) stay whole: a piece writes 25 to 64 KB that the merge reads
+// again, more than shorter heads gain (4 dense heads x 6000 x 96, 94 tiles: 50
+// us whole, 59 in pieces of 24; 4 dense heads on 1 x 64, 1000 rows of 10000
+// keys, 64 items of 157 tiles: 69 whole, 40 in pieces of 53).  Splitting a launch
 // that fills its rounds gains nothing, so the split plan is taken only where
 // its estimated time and the merge's, about 10 tiles, stay below the whole
 // one's.  D = 96, whole / in 2 to 4 splits: 32 dense heads, 1000 rows of 20000
@@ -773,8 +776,8 @@ static void plan_items(const msa_head_desc* heads, int H, int BH, int n_qb, int 
   const int cus = cus_per_xcd(), per_cu = wg_per_cu(D);
   const double slots = 8.0 * cus * per_cu;
   const double piece = fmax(total / slots / 2.0, D < 128 ? 64.0 : 32.0);
-  const double least = fmax(D < 128 ? 160.0 : 64.0, 1.5 * piece);
-  pl = ItemPlan();
+  const double least = fmax(D >= 128 ? 64.0 : n * n_qb <= 8 * cus ? 96.0 : 160.0, 1.5 * piece);
+  pl.clear();
   if (split && D <= 256 && longest > least) {
     for (int most = kMaxSplit; most > 1; --most) {
       int ns[kMaxHeads], entries = 0;
@@ -791,7 +794,7 @@ static void plan_items(const msa_head_desc* heads, int H, int BH, int n_qb, int 
     if (pl.n_sp && pick_ranges(pl.work, pl.n, n_qb, cus, per_cu, rg) + 10.0 <
                        pick_ranges(work, n, n_qb, cus, per_cu, rg))
       return;
-    pl = ItemPlan();
+    pl.clear();
   }
   for (int i = 0; i < n; ++i) pl.add(pairs[i], work[i], 1);
 }

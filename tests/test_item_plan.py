@@ -40,11 +40,13 @@ def test_full_rounds_stay_whole(D, S_k):
 
 def test_pieces_follow_each_head():
     """100 rows of 40000 keys: 625-tile heads in 8, 100-tile heads in 4 and
-    68-tile heads in 3 pieces of at most 32 tiles at D = 128; below it, 64-tile
-    pieces leave the sparse heads whole."""
+    68-tile heads in 3 pieces of at most 32 tiles at D = 128; below it pieces
+    have up to 64 tiles, the 68-tile heads stay whole, and the 100-tile heads
+    too once the items outnumber the CUs."""
     heads = [(DENSE, 0, 0)] * 3 + [(BLOCK, 100, 0)] * 19 + [(STREAM, 128, 4096)] * 10
     assert split_groups(heads, 100, 40000, 8, 128) == 3 * 8 + 19 * 4 + 10 * 3
-    assert split_groups(heads, 100, 40000, 8, 96) == 3 * 8
+    assert split_groups(heads, 100, 40000, 8, 96) == 3 * 8 + 19 * 2
+    assert split_groups(heads, 600, 40000, 8, 96) == 3 * 8
 
 
 def test_pieces_fit_the_list():
