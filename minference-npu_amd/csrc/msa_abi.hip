@@ -317,7 +317,7 @@ static bool k_can_stay(const msa_tensor4* k) {
   return D <= 256 && ss >= D && (s_pad * ss + D) * 2 <= (int64_t(1) << 31);
 }
 static bool k_stride_slow(const msa_tensor4* k) { return k->stride[2] % 64 != 32; }
-// what msa_stage_kv and every full prefill (S_q == S_k) leave in place
+// what msa_stage_kv and, for full prefills (S_q == S_k), msa_stage_kv_pool leave in place
 static bool k_in_place(const msa_tensor4* k) { return k_can_stay(k) && !k_stride_slow(k); }
 
 // Staging K pays where its tiles are read often enough: the copy takes about
@@ -327,26 +327,44 @@ static bool k_in_place(const msa_tensor4* k) { return k_can_stay(k) && !k_stride
 // 4 to 32 heads, groups of 1 and 4, in place / staged: D = 64, 17 reads 262 /
 // 274 us, 21 375 / 353, 31 832 / 816; D = 128, 8 reads 570 / 621, 14 873 / 884
 // and 277 / 257, 16 927 / 896, 28 455 / 399.
-static double k_reads_needed(int64_t D) { return D < 128 ? 28.0 : 12.0; }
-constexpr double kAllReads = 1e30;  // a full prefill: K of that size is a few MB
+static double k_reads_chunk(int64_t D) { return D < 128 ? 28.0 : 12.0; }
 
-// reads of a chunk's layer before its heads are known: those of sparse heads,
-// taken as 100 tiles a query block (top-k 100, or a window of 4096 keys and
-// sinks, 66)
-static double k_reads_sparse(const msa_tensor4* q, const msa_tensor4* k) {
-  if (q->size[2] == k->size[2]) return kAllReads;
-  return double(cdiv(q->size[2], MSA_BLOCK)) * double(q->size[1] / k->size[1]) *
-         fmin(1.0, 100.0 / double(cdiv(k->size[2], MSA_BLOCK)));
+// The same line for a full prefill (S_q == S_k) of `items` work items.
+// Measured on dense, unmasked and banded heads (256, 1024, 4096 keys), 2 to 32
+// of them, groups of 1 to 8, 300 to 16000 tokens, in place / staged:
+// - D = 64: a band of 256 keys (7 reads), 8 heads x 4000 17.9 / 20.3 us, of 1024
+//   (16) 24.8 / 26.7; from 30 reads on the staged K wins where the items fill
+//   the GPU's workgroups (8 dense x 4000, 32 reads, 504 items 39.7 / 37.9; 32
+//   heads x 8000, a band of 4096, 50 reads 281 / 270), not in smaller launches
+//   (2 x 8000, the same band, 250 items 34.6 / 36.4).
+// - D = 96 (rows of a fused projection) and 128: 7 reads 106 / 126 and 132 / 140
+//   (32 heads x 8000), 14 reads 52.9 / 48.8 and 63.8 / 58.5 (32 x 2000).
+// - D = 256: 7 reads 550 / 610 (32 x 16000), but 48.0 / 45.0 where the launch
+//   takes two rounds (2 x 16000, 500 items); 14 reads 116 / 111 (32 x 2000).
+static double k_reads_full(int64_t D, int64_t items) {
+  const int64_t cus = 8 * cus_per_xcd();
+  if (D < 96) return items >= cus * 7 / 4 ? 30.0 : 60.0;
+  return D > 128 && items > cus && items <= 2 * cus ? 0.0 : 8.0;
+}
+
+// Reads of a chunk's layer before its heads are known are those of sparse
+// heads, taken as 100 tiles a query block (top-k 100, or a window of 4096 keys
+// and sinks, 66).  In a full prefill K is staged by its stride alone there.
+static bool k_read_enough(const msa_tensor4* q, const msa_tensor4* k) {
+  return q->size[2] == k->size[2] ||
+         double(cdiv(q->size[2], MSA_BLOCK)) * double(q->size[1] / k->size[1]) *
+                 fmin(1.0, 100.0 / double(cdiv(k->size[2], MSA_BLOCK))) >=
+             k_reads_chunk(k->size[3]);
 }
 
 // The choice travels to the attention launch in the workspace.
-static int stage_k_mode(const msa_tensor4* k, double reads) {
+static int stage_k_mode(const msa_tensor4* k, bool read_enough) {
   if (!k_can_stay(k)) return 1;
-  return k_stride_slow(k) && reads >= k_reads_needed(k->size[3]) ? 1 : 0;
+  return k_stride_slow(k) && read_enough ? 1 : 0;
 }
 
-static int stage_setup(const msa_tensor4* k, const msa_tensor4* v, double k_reads, void* workspace,
-                       size_t workspace_bytes, StageParams& sp) {
+static int stage_setup(const msa_tensor4* k, const msa_tensor4* v, bool k_read_enough,
+                       void* workspace, size_t workspace_bytes, StageParams& sp) {
   if (!k || !v || !k->data || !v->data) return MSA_E_NULL;
   for (int i = 0; i < 4; ++i) {
     if (v->size[i] <= 0) return MSA_E_RANK;
@@ -377,7 +395,7 @@ static int stage_setup(const msa_tensor4* k, const msa_tensor4* v, double k_read
   sp.kv_heads = int(Hkv);
   sp.s_k = int(Sk);
   sp.s_pad = int(cdiv(Sk, MSA_BLOCK) * MSA_BLOCK);
-  sp.stage_k = stage_k_mode(k, k_reads);
+  sp.stage_k = stage_k_mode(k, k_read_enough);
   sp.k_flag = k_flag_of(workspace, need);
   return MSA_OK;
 }
@@ -391,7 +409,7 @@ static int stage_launch(const StageParams& sp, int dtype, int D, hipStream_t hs)
 int msa_stage_kv(const msa_tensor4* k, const msa_tensor4* v, void* workspace,
                  size_t workspace_bytes, msa_stream_t stream) {
   StageParams sp;
-  const int st = stage_setup(k, v, kAllReads, workspace, workspace_bytes, sp);
+  const int st = stage_setup(k, v, true, workspace, workspace_bytes, sp);
   if (st != MSA_OK) return st;
   return stage_launch(sp, v->dtype, int(v->size[3]), reinterpret_cast<hipStream_t>(stream));
 }
@@ -401,7 +419,7 @@ int msa_stage_kv_pool(const msa_tensor4* q, const msa_tensor4* k, const msa_tens
                       size_t est_workspace_bytes, void* workspace, size_t workspace_bytes,
                       msa_stream_t stream) {
   StageParams sp;
-  int st = stage_setup(k, v, kAllReads, workspace, workspace_bytes, sp);
+  int st = stage_setup(k, v, true, workspace, workspace_bytes, sp);
   if (st != MSA_OK) return st;
   if (n_slots > 0) {
     int16_t slot_kvp[kMaxHeads];
@@ -410,7 +428,7 @@ int msa_stage_kv_pool(const msa_tensor4* q, const msa_tensor4* k, const msa_tens
                     slot_kvp, L);
     if (st != MSA_OK) return st;
     sp.n_pool_wg = pool_workgroups(sp.pool);
-    sp.stage_k = stage_k_mode(k, k_reads_sparse(q, k));
+    sp.stage_k = stage_k_mode(k, k_read_enough(q, k));
   } else if (n_slots < 0) {
     return MSA_E_HEADS;
   }
@@ -580,19 +598,24 @@ static double prefix_cost(const HeadWork& w, double m) {
   return tiles / w.div + w.fixed * m;
 }
 
-// reads of K (k_reads_sparse) by the heads of a layer
-static double k_reads(const msa_tensor4* q, const msa_tensor4* k, const msa_head_desc* heads,
-                      int topk_max) {
-  if (q->size[2] == k->size[2]) return kAllReads;
+// the same with the heads of the layer; yes with vertical_and_slash heads,
+// whose launch counts on K staged by its stride
+static bool k_read_enough(const msa_tensor4* q, const msa_tensor4* k, const msa_head_desc* heads,
+                          int topk_max) {
   const int n_qb = int(cdiv(q->size[2], MSA_BLOCK)), n_kb = int(cdiv(k->size[2], MSA_BLOCK));
   double tiles = 0.0;
+  int64_t items = 0;
   for (int h = 0; h < int(q->size[1]); ++h) {
     if (heads[h].kind == MSA_KIND_SKIP) continue;
+    if (heads[h].kind == MSA_KIND_VS) return true;
     HeadWork w = head_work(heads[h], n_qb, n_kb, topk_max);
     w.fixed = 0.0;
     tiles += prefix_cost(w, n_qb);
+    items += q->size[0] * n_qb;
   }
-  return tiles / (double(n_kb) * double(k->size[1]));
+  const double line = q->size[2] == k->size[2] ? k_reads_full(k->size[3], items)
+                                               : k_reads_chunk(k->size[3]);
+  return tiles >= line * double(n_kb) * double(k->size[1]);
 }
 
 // attention workgroups that share a CU (not vertical_and_slash)
@@ -896,7 +919,7 @@ static int layer_attention_impl(const msa_tensor4* q, const msa_tensor4* k, cons
   hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
   if (stage) {
     StageParams sp;
-    st = stage_setup(k, v, k_reads(q, k, heads, topk_max), workspace, workspace_bytes, sp);
+    st = stage_setup(k, v, k_read_enough(q, k, heads, topk_max), workspace, workspace_bytes, sp);
     if (st == MSA_OK) st = stage_launch(sp, v->dtype, D, hs);
     if (st != MSA_OK) return st;
   }
@@ -1024,7 +1047,7 @@ static int layer_attention_impl(const msa_tensor4* q, const msa_tensor4* k, cons
     // the vertical_and_slash kernel reads staged K: stage the K the plain
     // staging left in place (V and its exponents are staged already)
     StageParams kp;
-    st = stage_setup(k, v, kAllReads, workspace, workspace_bytes, kp);
+    st = stage_setup(k, v, true, workspace, workspace_bytes, kp);
     if (st != MSA_OK) return st;
     kp.stage_k = 2;
     kp.k_flag = nullptr;  // the other heads' launch still reads K in place
