@@ -87,3 +87,34 @@ def test_many_pairs_plain_order(gpu_device):
     """More (batch, head) pairs than one item list: the plain item order."""
     q, k, v = (t.to(gpu_device) for t in make_qkv(17, 8, 65, 65, 128, torch.bfloat16, seed=17))
     assert _layer(gpu_device, q, k, v, 65) < TOL
+
+
+@pytest.mark.parametrize("D", [96, 128, 256])
+@pytest.mark.parametrize("j", [0, 63, 150, 299])
+def test_non_finite_keys_and_values(gpu_device, D, j):
+    """A NaN key reaches the rows that see it and no other; an infinite V its
+    own dim of them."""
+    from minference.backend.attention import dense_attention
+
+    g = torch.Generator().manual_seed(j + D)
+    q, k, v = (torch.randn(1, 2, 300, D, generator=g).half() for _ in range(3))
+    mask = torch.ones(300, 300, dtype=torch.bool).tril()
+    ref = torch.nn.functional.scaled_dot_product_attention(q.float(), k.float(), v.float(),
+                                                           attn_mask=mask)
+
+    def run(k, v):
+        out = torch.empty(q.shape, device=gpu_device)
+        return dense_attention(*(t.to(gpu_device) for t in (q, k, v)), out=out).cpu()
+
+    bad = k.clone()
+    bad[:, :, j, 3] = float("nan")
+    out = run(bad, v)
+    assert torch.isnan(out[:, :, j:]).all()
+    if j:
+        assert float((out - ref)[:, :, :j].abs().max()) < TOL
+    bad = v.clone()
+    bad[:, :, j, 9] = float("inf")
+    out = run(k, bad)
+    assert (out[:, :, j:, 9] == float("inf")).all()
+    out[..., 9] = ref[..., 9]
+    assert float((out - ref).abs().max()) < 2 * TOL  # |V| < 6 here: 2^-11 of 6
