@@ -299,13 +299,14 @@ static int cus_per_xcd() {
 
 // The attention kernel reads K in place, from the caller's rows, when every
 // offset of one kv head's padded rows fits 31 bits, the rows do not overlap
-// and the row stride is an odd multiple of 64 bytes; otherwise the staging
-// writes K in operand order first.  An in-place operand load reads 64 bytes
-// of each of 16 rows, four rows per group of four lanes: with L2-resident
-// rows such loads run at 38 B/ns per CU when the stride is a multiple of 128
-// bytes (the four rows meet in one L1 bank; head dims 64, 128 and 256, and
-// every view of a fused projection) and at 75 B/ns when it is an odd multiple
-// of 64 (contiguous rows of 96), against 134 B/ns for a staged operand's
+// and either the row stride is an odd multiple of 64 bytes or the launch reads
+// each tile a few times only (k_reads_chunk, k_reads_full); otherwise the
+// staging writes K in operand order first.  An in-place operand load reads 64 bytes
+// of each of 16 rows, four rows per group of four lanes: in a probe of such
+// loads on L2-resident rows they ran at 38 B/ns per CU when the stride is a
+// multiple of 128 bytes (head dims 64, 128 and 256, and every view of a fused
+// projection; why was not measured) and at 75 B/ns when it is an odd multiple of
+// 64 (contiguous rows of 96), against 134 B/ns for a staged operand's
 // contiguous 1 KB.  At 38 B/ns the K loads alone fill the kernel's time:
 // attention module of a fused projection, 32 heads x 96, 16000 tokens, 2530
 // us in place and 2270 us staged (8000 tokens: 1081 and 1002); contiguous

@@ -527,7 +527,9 @@ __device__ inline void lds_barrier() {
 // rows cost 4 D / 32 loads per wave at 38 or 75 B/ns per CU, 1 to 2 us of the
 // L1 per item.  Before -> after: block ids at 32K of D = 128, short items, 255
 // -> 241 us; stream 16K of D = 256 604 -> 586; causal 8000 of D = 128 304 ->
-// 301; the 64K layer of D = 96, long items, 4508 -> 4479.
+// 301; the 64K layer of D = 96, long items, 4433 -> 4405; 440 launches of D = 64
+// and 96, 64 to 9000 tokens, 1 to 2 % in the median and up to 9 %, seven of them
+// the other way by 2 to 3 %.
 template <int D>
 struct QTile {
   static constexpr int NKS = D / 32;
@@ -1179,9 +1181,10 @@ void attn_kernel(AttnParams P) {
 // 2^15 leaves the tile's stamp in LDS, and after the tile's barrier every
 // wave takes the rare path together (row maxima exchanged through LDS, O and
 // sums rescaled, P written again).
-// Registers: 243 at D = 128 (two waves per SIMD), 426 at D = 256 (one).
-// Bound by the waits between the phases of a tile (MFMA busy 46 % of the
-// cycles at D = 128, 1.87 GHz).  With the staged K (k_in_place in msa_abi.hip),
+// Registers: 254 at D = 128 (two waves per SIMD), 428 at D = 256 (one).
+// Bound by the waits between the phases of a tile: MFMA busy 44 % of the
+// cycles at D = 128 (dense 8000, 1.78 GHz; 31 % on 17-tile items), 38 % at D =
+// 256 (2.08 GHz); LDS conflicts stall 1 % at most.  With the staged K (k_in_place in msa_abi.hip),
 // whole calls against attn_kernel (D = 128) and a kernel with 16 rows per wave
 // and each tile copied to LDS (D = 256): dense fp16, 16 heads x 8000 x 128,
 // 362 -> 310 us; one 16K layer of 32 heads on 8 kv heads x 128, 1543 ->

@@ -203,7 +203,11 @@ static hipError_t launch_rope_t(const RopeParams& p, int dtype, hipStream_t st) 
 // with many, fewer tokens per block only read the tables more often.  Launch
 // times, 32 + 32 heads x 96, 16 / 4 / 1 tokens: 512 tokens 17.6 / 7.8 / 7.5 us,
 // 1000 18.4 / 8.8 / 11.9, 2000 19.5 / 14.7 / 21.7, 4000 22.2 / 24.9 / 37.9,
-// 32768 163 / 184 / 362.
+// 32768 163 / 184 / 362.  16 tokens / the rule's at 2500, 3000 and 3071 tokens:
+// 32 + 8 heads x 128 16.4 / 14.2, 16.3 / 15.4, 16.4 / 15.6; 8 + 2 x 128 10.0 /
+// 6.2, 10.2 / 6.5, 10.2 / 6.4; 128 + 8 x 128 36.7 / 32.3, 37.1 / 35.7, 39.0 /
+// 36.2; 64 + 8 x 128, whose 18 head groups take a block's 16 waves twice, 22.6 /
+// 21.8, 23.0 / 23.8, 22.9 / 24.1.
 hipError_t launch_rope(const RopeParams& p, int dtype, hipStream_t st) {
   const int64_t n_tok = int64_t(p.batch) * p.s;
   if (n_tok >= 3072) return launch_rope_t<16>(p, dtype, st);

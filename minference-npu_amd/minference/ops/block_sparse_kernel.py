@@ -162,8 +162,10 @@ def _attend_ids(q, k, v, ids, bs, out):
 
 
 def tile_ids(block_indices: torch.Tensor, block_size: int, n_qb: int) -> torch.Tensor:
-    """The first half of msa_block_lists in torch ops (any device): ids of ``block_size``-token blocks [B, H, n_q_blocks, topk] as ids of
-    the kernels' 64-token tiles [B, H, n_qb, topk * m] (m = block_size / 64):
+    """The first half of msa_block_lists in torch ops, on any device (the
+    attention calls take the launch; this form is what it is compared with):
+    ids of ``block_size``-token blocks [B, H, n_q_blocks, topk] as ids of the
+    kernels' 64-token tiles [B, H, n_qb, topk * m] (m = block_size / 64):
     block J is tiles m J .. m J + m - 1, and 64-row query block bq takes the
     list of its block bq // m.  The token visibility is unchanged: a key is
     in a selected block iff its tile is among that block's tiles.  Ids
@@ -176,8 +178,9 @@ def tile_ids(block_indices: torch.Tensor, block_size: int, n_qb: int) -> torch.T
 
 
 def canonical_block_lists(block_indices: torch.Tensor, n_kb: int):
-    """The second half of msa_block_lists in torch ops (any device): turn
-    arbitrary per-row block ids into the kernel's list format: the distinct ids in [0, n_kb) ascending first, ``cnt`` = how many.  This is the
+    """The second half of msa_block_lists in torch ops, on any device (see
+    tile_ids): arbitrary per-row block ids in the kernel's list format, the
+    distinct ids in [0, n_kb) ascending first, ``cnt`` = how many.  This is the
     set semantics of the reference's scatter into a block mask
     (block_sparse_kernel_npu.py:290-291): repeats count once and ids outside
     the key range select nothing.  Returns int32 (idx, cnt)."""
