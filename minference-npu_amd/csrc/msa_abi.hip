@@ -775,7 +775,9 @@ struct ItemPlan {
 // have a CU each) stay whole: a piece writes 25 to 64 KB that the merge reads
 // again, more than shorter heads gain (4 dense heads x 6000 x 96, 94 tiles: 50
 // us whole, 59 in pieces of 24; 4 dense heads on 1 x 64, 1000 rows of 10000
-// keys, 64 items of 157 tiles: 69 whole, 40 in pieces of 53).  Splitting a launch
+// keys, 64 items of 157 tiles: 69 whole, 40 in pieces of 53; 185 such launches
+// with heads of 97 to 112 tiles, whole over cut: median 1.20, nine below 0.98, 2
+// heads of 8000 x 96 least, 50.4 / 55.5).  Splitting a launch
 // that fills its rounds gains nothing, so the split plan is taken only where
 // its estimated time and the merge's, about 10 tiles, stay below the whole
 // one's.  D = 96, whole / in 2 to 4 splits: 32 dense heads, 1000 rows of 20000
